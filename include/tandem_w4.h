@@ -64,7 +64,7 @@ int tw4_init(int device);
 /* AutoAWQ "gemm" tensors -> tile layout, on the device.
  *   qweight int32 [K, N/8], qzeros int32 [K/128, N/8] (AWQ nibble order 0,2,4,6,1,3,5,7),
  *   scales fp16 [K/128, N]  ->  packed [Npad/16 * K/128 * 256] int32, scales_out / zeros_out
- *   fp16 [N, K/128]. packed must be zero-filled by the caller (its rows >= N stay zero).
+ *   fp16 [N, K/128]. Every word of packed is written, its rows >= N with zeros.
  * interleave = 1 reorders rows as interleave_gate_up (gate rows 8T..8T+7 then up rows
  * N/2+8T..N/2+8T+7 in row tile T; N % 16 == 0).
  * Replaces repack_awq + interleave_gate_up (python/tandem/layers/awq.py:42-75, 235-241). */

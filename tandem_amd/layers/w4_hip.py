@@ -336,7 +336,7 @@ def repack(qweight: torch.Tensor, qzeros: torch.Tensor, scales: torch.Tensor,
                          f"scales {tuple(scales.shape)} group 128")
     qweight, qzeros, scales = qweight.contiguous(), qzeros.contiguous(), scales.contiguous()
     dev = qweight.device
-    packed = torch.zeros((padded_rows(n), k // 8), dtype=torch.int32, device=dev)
+    packed = torch.empty((padded_rows(n), k // 8), dtype=torch.int32, device=dev)  # padding rows too are written
     s_out = torch.empty((n, k // 128), dtype=torch.float16, device=dev)
     z_out = torch.empty((n, k // 128), dtype=torch.float16, device=dev)
     with torch.cuda.device(dev):
