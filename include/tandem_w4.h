@@ -61,6 +61,10 @@ const char* tw4_last_error(void);
  * (python/tandem/layers/awq.py:247-251). Safe to call repeatedly. */
 int tw4_init(int device);
 
+/* A number of the HIP graph capture `stream` is part of, the same for every call within one capture and different for
+ * every other (0: none is going on), by which a caller keeps a workspace per captured graph. No reference counterpart. */
+uint64_t tw4_capture_id(void* stream);
+
 /* AutoAWQ "gemm" tensors -> tile layout, on the device.
  *   qweight int32 [K, N/8], qzeros int32 [K/128, N/8] (AWQ nibble order 0,2,4,6,1,3,5,7),
  *   scales fp16 [K/128, N]  ->  packed [Npad/16 * K/128 * 256] int32, scales_out / zeros_out
@@ -200,6 +204,21 @@ int tw4_gemm(const uint16_t* x, const int32_t* packed, const uint16_t* scales,
              int64_t ws_floats, int64_t n_locks, int M, int N, int K,
              int mt, int nt, int warps_n, int warps_k, int stages, int splits, int act,
              void* stream);
+
+/* tw4_gemm's stages-3 kernel (both tiles through LDS) with every tile and ring depth it is compiled for, and for any
+ * N % 8 == 0 with scales and zeros 4-byte aligned. BM = 16 mt warps_m tokens, BN = 16 nt warps_n rows, `ring` stages
+ * of 64 k in LDS, warps_k 1, or 2: two wavefronts per (tokens, rows) part, each with half of every stage. splits: 0 as
+ * for stages 3, 1, or that many contiguous ranges of whole quant groups per tile (at most 2 K / 128; a range past the
+ * groups is empty). Otherwise tw4_gemm's contract. No reference counterpart
+ * beyond w4_gemm's (python/tandem/csrc/w4_gemv.cu:312-566). */
+int tw4_gemm_tiled(const uint16_t* x, const int32_t* packed, const uint16_t* scales,
+                   const uint16_t* zeros, uint16_t* y, float* ws, int32_t* locks,
+                   int64_t ws_floats, int64_t n_locks, int M, int N, int K,
+                   int mt, int nt, int warps_n, int warps_m, int warps_k, int ring, int splits, int act,
+                   void* stream);
+
+/* Compiled (mt, nt, warps_n, warps_m, warps_k, ring) configurations of tw4_gemm_tiled; returns how many. */
+int tw4_gemm_tiled_configs(int* out, int max_configs);
 
 /* tw4_gemm without a caller workspace, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc). No counterpart in the

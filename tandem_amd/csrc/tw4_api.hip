@@ -62,3 +62,12 @@ extern "C" int tw4_init(int device) {
     }
     return rc;
 }
+
+extern "C" uint64_t tw4_capture_id(void* stream) {
+    if (!stream) return 0;  // the null stream is never captured
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &id) != hipSuccess) return 0;
+    // never 0 for an active capture
+    return status == hipStreamCaptureStatusActive ? static_cast<uint64_t>(id) + 1 : 0;
+}

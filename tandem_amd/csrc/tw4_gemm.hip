@@ -595,11 +595,17 @@ int tw4_gemm_lds_dispatch(const uint16_t* x, const int32_t* packed, const uint16
                           uint16_t* y, float* ws, int32_t* locks, int64_t ws_floats, int64_t n_locks, int M, int N,
                           int K, int mt, int nt, int warps_n, int warps_m, int splits, int cus, int act, void* stream);
 int tw4_gemm_lds_configs(int* out, int max_configs, int start);
+int tw4_gemm_tiled_dispatch(const uint16_t* x, const int32_t* packed, const uint16_t* scales, const uint16_t* zeros,
+                            uint16_t* y, float* ws, int32_t* locks, int64_t ws_floats, int64_t n_locks, int M, int N,
+                            int K, int mt, int nt, int warps_n, int warps_m, int warps_k, int ring, int splits, int cus,
+                            int act, void* stream);
 
-extern "C" int tw4_gemm(const uint16_t* x, const int32_t* packed, const uint16_t* scales, const uint16_t* zeros,
-                        uint16_t* y, float* ws, int32_t* locks, int64_t ws_floats, int64_t n_locks, int M, int N,
-                        int K, int mt, int nt, int warps_n, int warps_k, int stages, int splits, int act,
-                        void* stream) {
+namespace {
+
+// The argument checks every GEMM entry point shares, and the device's set-up (index in dev).
+int gemm_check(const uint16_t* x, const int32_t* packed, const uint16_t* scales, const uint16_t* zeros, const uint16_t* y,
+               const float* ws, const int32_t* locks, int64_t ws_floats, int64_t n_locks, int M, int N, int K, int splits,
+               int act, int& dev) {
     TW4_REQUIRE(x && packed && scales && zeros && y, TW4_EINVAL, "gemm: null pointer");
     TW4_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0, TW4_EINVAL, "gemm: x must be 16-byte aligned");
     TW4_REQUIRE(reinterpret_cast<uintptr_t>(packed) % 16 == 0, TW4_EINVAL, "gemm: packed must be 16-byte aligned");
@@ -612,15 +618,36 @@ extern "C" int tw4_gemm(const uint16_t* x, const int32_t* packed, const uint16_t
     TW4_REQUIRE(splits >= 0 && splits <= 16, TW4_EINVAL, "gemm: splits 0 (split the last wave) or 1 .. 16");
     TW4_REQUIRE(splits <= 1 || (ws && locks), TW4_EINVAL, "gemm: split-K needs a workspace and counters");
     TW4_REQUIRE(ws_floats >= 0 && n_locks >= 0, TW4_EINVAL, "gemm: workspace sizes must be >= 0");
-    ws_floats = ws_floats < kMaxPartialFloats ? ws_floats : kMaxPartialFloats;  // the part split-K may use
     if (M == 0) return TW4_OK;
-    int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return tw4host::hip_fail(e, "gemm: hipGetDevice");
-    if (dev < 0 || dev >= kMaxDevices || !g_dev[dev].ready) {
-        int rc = device_prepare(dev);
-        if (rc) return rc;
-    }
+    if (dev < 0 || dev >= kMaxDevices || !g_dev[dev].ready) return device_prepare(dev);
+    return TW4_OK;
+}
+
+}  // namespace
+
+extern "C" int tw4_gemm_tiled(const uint16_t* x, const int32_t* packed, const uint16_t* scales, const uint16_t* zeros,
+                              uint16_t* y, float* ws, int32_t* locks, int64_t ws_floats, int64_t n_locks, int M, int N,
+                              int K, int mt, int nt, int warps_n, int warps_m, int warps_k, int ring, int splits, int act,
+                              void* stream) {
+    int dev = 0;
+    const int rc = gemm_check(x, packed, scales, zeros, y, ws, locks, ws_floats, n_locks, M, N, K, splits, act, dev);
+    if (rc || M == 0) return rc;
+    if (splits == 0 && !(ws && locks)) splits = 1;
+    return tw4_gemm_tiled_dispatch(x, packed, scales, zeros, y, ws, locks,
+                                   ws_floats < kMaxPartialFloats ? ws_floats : kMaxPartialFloats, n_locks, M, N, K, mt, nt,
+                                   warps_n, warps_m, warps_k, ring, splits, g_dev[dev].cus, act, stream);
+}
+
+extern "C" int tw4_gemm(const uint16_t* x, const int32_t* packed, const uint16_t* scales, const uint16_t* zeros,
+                        uint16_t* y, float* ws, int32_t* locks, int64_t ws_floats, int64_t n_locks, int M, int N,
+                        int K, int mt, int nt, int warps_n, int warps_k, int stages, int splits, int act,
+                        void* stream) {
+    int dev = 0;
+    const int rc = gemm_check(x, packed, scales, zeros, y, ws, locks, ws_floats, n_locks, M, N, K, splits, act, dev);
+    if (rc || M == 0) return rc;
+    ws_floats = ws_floats < kMaxPartialFloats ? ws_floats : kMaxPartialFloats;  // the part split-K may use
     if (splits == 0 && !(ws && locks)) splits = 1;
     if (stages == 1)
         return tw4_gemm_mid_dispatch(x, packed, scales, zeros, y, ws, locks, ws_floats, n_locks, M, N, K, mt, nt,

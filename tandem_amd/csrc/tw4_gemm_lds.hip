@@ -1,262 +1,313 @@
-// Fused-dequant GEMM for large M (prefill): y[M, N] = x[M, K] @ dequant(W)^T, with BOTH operand
-// tiles staged through LDS by gfx950's direct-to-LDS loads (global_load_lds_dwordx4), a 3-deep ring.
+// Fused-dequant GEMM for M > 16: y[M, N] = x[M, K] @ dequant(W)^T, with BOTH operand tiles staged through LDS by
+// gfx950's direct-to-LDS loads (buffer_load ... lds), a ring of R slots.
 //
-// Workgroup tile BM x BN = (WM wavefronts x 16 MT tokens) x (WN wavefronts x 16 NT rows); wavefront
-// (wm, wn) computes 16 MT tokens x 16 NT rows. A stage is half a quant group (BK = 64 k): stage s
-// covers k = 64 s .. 64 s + 63 of group s / 2.
-//   x:       the BM x 64 fp16 tile, 128 B per token row, 8 rows per load instruction. LDS slot
-//            (row rho, position p) holds 16-byte chunk p ^ ((rho >> 1) & 7) of the row. Two rows fill
-//            the 64 banks, even rows the lower 32, odd rows the upper 32; the swizzle gives the 8
-//            even (and the 8 odd) rows of a B-fragment read (16 rows, one chunk) 8 different 16-byte
-//            positions, so its 16 lanes touch every bank once (with rho & 7, each position came
-//            twice: a 2-way bank conflict on every x read).
-//   weights: the int4 tile as it sits in HBM: the k half of each (row tile, group) 1 KB block is 512
-//            contiguous bytes (words kb = 2 h, 2 h + 1 of [kb][r][s]), two row tiles per instruction.
-//            Every weight byte is read from HBM once per workgroup; the WM wavefronts that share a
-//            row tile each read it from LDS as int4 (a quarter of the fp16 bytes) and dequantize the
-//            words they need in registers.
+// Workgroup tile BM x BN = (WM wavefronts x 16 MT tokens) x (WN wavefronts x 16 NT rows); wavefront (wm, wn) computes
+// 16 MT tokens x 16 NT rows, over all of K or (WK = 2) two wavefronts over one of the two 32-k substeps of every stage
+// each, added in LDS at the end. A stage is half a quant group (BK = 64 k): stage s covers k = 64 s .. 64 s + 63 of
+// group s / 2.
+//   x:       the BM x 64 fp16 tile, 128 B per token row, 8 rows per load instruction. LDS slot (row rho, position p)
+//            holds 16-byte chunk p ^ ((rho >> 1) & 7) of the row. Two rows fill the 64 banks, even rows the lower 32,
+//            odd rows the upper 32; the swizzle gives the 8 even (and the 8 odd) rows of a B-fragment read (16 rows, one
+//            chunk) 8 different 16-byte positions, so its 16 lanes touch every bank once.
+//   weights: the int4 tile as it sits in HBM: the k half of each (row tile, group) 1 KB block is 512 contiguous bytes
+//            (words kb = 2 h, 2 h + 1 of [kb][r][s]), two row tiles per instruction. Every weight byte is read from
+//            HBM once per workgroup; the WM wavefronts that share a row tile each read it from LDS as int4 (a quarter
+//            of the fp16 bytes) and dequantize the words they need in registers.
 //   params:  each wavefront's NT tiles' 16 scales and 16 zeros of the group (64 B per tile).
-//   math:    v_mfma_f32_16x16x32_f16, A = dequantized weights fp16_rne((q - z) s) (16 rows x 32 k),
-//            B = x (32 k x 16 tokens). Substep j (0, 1) of a stage: lane (q, r) feeds A row r and B
-//            column r the k values of word (kb = 2 h + (q >> 1), s = 2 j + (q & 1)), i.e.
-//            k = 64 s + 32 (q >> 1) + 16 j + 8 (q & 1) + 0..7, the same permutation for both operands.
+//   math:    v_mfma_f32_16x16x32_f16, A = dequantized weights fp16_rne((q - z) s) (16 rows x 32 k), B = x (32 k x 16
+//            tokens). Substep j (0, 1) of a stage: lane (q, r) feeds A row r and B column r the k values of word
+//            (kb = 2 h + (q >> 1), s = 2 (q & 1) + j), i.e. k = 64 s + 32 (q >> 1) + 16 (q & 1) + 8 j + 0..7, the same
+//            permutation for both operands: a lane's two words of a stage are one 8-byte read.
 //            D lane (q, r) = rows 4 q + i of token r, the layout finish_unit stores.
-//   ring:    R = 3 or 4 slots. Stage i waits for its own loads (vmcnt), one workgroup barrier, issues
-//            stage i + R - 1 into the slot stage i - 1 used, then computes from LDS, so R - 1 stages of
-//            loads are in flight under every stage's math.
-//   split-K: work units (tile, split) take contiguous stage ranges; the epilogue is the other GEMM's
+//   ring:    R slots. At stage i + 1's start the wavefront waits for its own loads of it (vmcnt), the workgroup meets,
+//            and stage i's slot takes the loads of stage i + R, so R - 2 or more stages of loads are in flight.
+//   split-K: work units (tile, split) take contiguous ranges of whole groups; the epilogue is the other GEMM's
 //            finish_unit (deterministic last-arriver reduction, counters returned to zero).
-#include "tw4_common.h"
+//
+// What bounds it. Long calls (M N K from about 2^36): the matrix core, at the clock the card's power allows (1.7-1.9 GHz
+// under this load); 1.24 PFLOP/s against 1.3-1.5 of hipBLASLt's fp16 product without the dequantization. A wavefront
+// issues in order, about one instruction in 4 cycles, and an MFMA takes 16: the loop is software-pipelined in registers
+// (the next fragments are read and the next weights dequantized between the current MFMAs, substep below), where a
+// read - dequantize - multiply sequence per substep left the matrix core idle for the first two. Short calls: the wait
+// for the first stages, the number of stages a CU runs in a row and how evenly the tiles divide over the CUs, hence the
+// small tiles with WK = 2, two workgroups per CU and K splits. Before -> after, us, the same sizes (K x N, M), weights
+// streamed from HBM: 4096 x 6144, 512: 48 -> 32; 4096 x 24576, 128 / 256 / 512: 43 / 78 / 105 -> 33 / 56 / 95;
+// 12288 x 4096, 512: 66 -> 60; 4096 x 28672, 77: 48 -> 30; 5120 x 34816, 40 / 2048: 133 / 722 -> 37 / 600 (the last one
+// dequantized + hipBLASLt before).
+#include "tw4_lds.h"
 
 namespace tw4 {
 
-typedef __attribute__((address_space(3))) const void lds_void;
-
-// Direct-to-LDS load of BYTES (4 or 16) per lane: lane l's BYTES at global `src` go to LDS byte address
-// `lds_addr` (wavefront-uniform) + l BYTES. Issued as inline assembly so that the compiler, which cannot tell the
-// ring's slots apart for these loads, does not add a wait for every load in flight before each LDS
-// read; the ring waits with explicit vmcnt counts instead, and the loop holds no other vector memory
-// operation. M0 (the LDS base operand) is saved and restored around the load, one wait state after
-// writing it (the M0 -> LDS-DMA hazard).
-// The global address is a wavefront-uniform 64-bit base in SGPRs (`sbase`, the part that moves with the
-// stage) plus this lane's 32-bit byte offset `voff` (fixed for the whole kernel), the instruction's
-// scalar-base form: no per-lane 64-bit address arithmetic per load.
-template <int BYTES>
-__device__ __forceinline__ void lds_dma(const void* sbase, uint32_t voff, uint32_t lds_addr) {
-    const uint32_t base = __builtin_amdgcn_readfirstlane(lds_addr);
-    uint32_t saved;
-    if constexpr (BYTES == 16)
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b32 m0, %0"
-                     : "=&s"(saved) : "v"(voff), "s"(sbase), "s"(base) : "memory");
-    else
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %3\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2\n\ts_mov_b32 m0, %0"
-                     : "=&s"(saved) : "v"(voff), "s"(sbase), "s"(base) : "memory");
+// Pair i (weights 2 i, 2 i + 1) of a word, dequantized: dequant_word in quarters.
+__device__ __forceinline__ h2 dequant_pair(uint32_t w, int i, const GroupQ& p, uint32_t magic) {
+    const h2 sixteenth = h2{static_cast<h1>(0.0625f), static_cast<h1>(0.0625f)};
+    const uint32_t v = i < 2 ? w : w >> 8;
+    if (i & 1) return (bitcast<h2>((v & 0x00F000F0u) | magic) * sixteenth + p.zhi) * p.s;
+    return (bitcast<h2>((v & 0x000F000Fu) | magic) + p.zlo) * p.s;
 }
 
-template <int MT, int NT, int WM, int WN>
+#define TW4_STEP_FENCE __builtin_amdgcn_sched_barrier(0)
+
+// acc += A B on v_mfma_f32_16x16x32_f16 with the accumulator held in accumulation registers for the whole loop: left
+// to the compiler, the loop's accumulators move between the two register files at every iteration. FIRST: the first
+// of a step, two wait states after the vector instructions that wrote A.
+template <bool FIRST>
+__device__ __forceinline__ void mfma_acc(f4& c, const h8& a, const h8& b) {
+    if constexpr (FIRST)
+        asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+    else
+        asm volatile("v_mfma_f32_16x16x32_f16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+
+// The accumulators after the loop's last MFMA: 32 wait states (16x16x32 needs 18 before a vector read of its result),
+// after which they are ordinary values again.
+template <int NT, int MT>
+__device__ __forceinline__ void mfma_settle(f4 (&acc)[NT][MT]) {
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int b = 0; b < MT; ++b) asm volatile("" : "+a"(acc[t][b]));
+}
+
+template <int MT_, int NT_, int WM_, int WN_, int WK_, int R_>
 struct LdsGemmCfg {
+    static constexpr int MT = MT_, NT = NT_, WM = WM_, WN = WN_, WK = WK_, R = R_;
     static constexpr int BM = 16 * MT * WM;
     static constexpr int BN = 16 * NT * WN;
-    static constexpr int WAVES = WM * WN;
+    static constexpr int WAVES = WM * WN * WK;
     static constexpr int THREADS = 64 * WAVES;
     static constexpr int X_U4 = BM * 8;               // x tile: BM rows x 8 chunks
     static constexpr int W_U4 = BN / 16 * 32;         // weights: BN / 16 half-blocks of 512 B
-    static constexpr int P_U4 = WAVES * 32;           // params: per wavefront 8 tiles' 16 scales, then their zeros
+    static constexpr int P_INSTR = NT <= 4 ? 1 : 2;   // params loads per wavefront and group (256 B each)
+    static constexpr int P_U4 = WAVES * 16 * P_INSTR; // per wavefront its tiles' 16 scales each, then their zeros
     static constexpr int SLOT_U4 = X_U4 + W_U4 + P_U4;
-    static constexpr int X_INSTR = BM / 8 / WAVES;    // x loads per wavefront per stage (8 rows each)
-    static constexpr int W_INSTR = BN / 32 / WAVES;   // weight loads per wavefront per stage (2 half-blocks)
-    static constexpr int P_INSTR = 2;                 // params loads per wavefront: scales, zeros (8 tiles x 32 B)
-    static constexpr int LOADS = X_INSTR + W_INSTR + P_INSTR;
-    // registers for two wavefronts per SIMD (at most 256 each) where the accumulators allow it and two
-    // wavefronts per SIMD can be resident: 8 wavefronts per workgroup, or 4 with a ring small enough
-    // (BM = 128) that two workgroups share a CU and run out of phase
-    static constexpr int MIN_WAVES_PER_SIMD = MT * NT <= 32 && (WAVES >= 8 || BM <= 128) ? 2 : 1;
-    static_assert(BM % (8 * WAVES) == 0, "x rows split evenly over the wavefronts");
-    static_assert(BN % (32 * WAVES) == 0, "weight half-blocks split evenly over the wavefronts");
-    static_assert(NT == 4 || NT == 8, "params: one dword load covers 8 tiles' 16 values (NT = 4 loads 4 twice)");
-    static_assert(3 * LOADS < 64, "s_waitcnt vmcnt immediate");
+    static constexpr int X_LOADS = BM / 8;            // 1 KB loads of a stage: 8 token rows each
+    static constexpr int W_LOADS = BN / 32;           // two half-blocks each
+    static constexpr int X_INSTR = (X_LOADS + WAVES - 1) / WAVES;  // per wavefront (the last ones may repeat a load)
+    static constexpr int W_INSTR = (W_LOADS + WAVES - 1) / WAVES;
+    static constexpr int XW = X_INSTR + W_INSTR;
+    static constexpr int LDS_BYTES = R * SLOT_U4 * 16;
+    // wavefronts per SIMD the registers are kept for: two where the accumulators leave room for it and two
+    // workgroups fit a CU's 160 KB of LDS (or the workgroup itself has eight wavefronts)
+    static constexpr int MIN_WAVES_PER_SIMD = MT * NT <= 32 && (WAVES >= 8 || LDS_BYTES <= 80 * 1024 - 256) ? 2 : 1;
+    static_assert(WK == 1 || (WK == 2 && WM * WN * MT * NT * 64 <= R * SLOT_U4), "the K halves' sums fit the ring");
+    static_assert(R >= 3, "ring of at least 3 slots");
+    static_assert(BM % 8 == 0 && BN % 32 == 0, "whole 1 KB loads");
+    static_assert(NT >= 2 && NT <= 8, "params: one dword load covers 4 tiles' scales and zeros, or 8 tiles' of one");
+    static_assert((R - 1) * (XW + P_INSTR) < 64, "s_waitcnt vmcnt immediate");
+    static_assert(LDS_BYTES <= 160 * 1024 - 64, "one workgroup's LDS");
 };
 
-// s_waitcnt with only vmcnt limited (expcnt and lgkmcnt at their maxima); gfx9's 6-bit vmcnt is
-// split over bits 3:0 and 15:14 of the immediate.
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt immediate");
-    __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x70 | 0xF00);
-}
-
-// A workgroup barrier that orders no memory by itself (the LDS data it guards was waited for with
-// wait_vmcnt): s_barrier between two compiler-only fences, so no LDS access moves across it.
-__device__ __forceinline__ void ring_barrier() {
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    __builtin_amdgcn_s_barrier();
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-}
-
-template <int MT, int NT, int WM, int WN>
+template <class C>
 struct LdsGemmArgs {
-    using C = LdsGemmCfg<MT, NT, WM, WN>;
-    const char* x;  // byte bases; a stage adds its k offset to them (scalar) and each lane its offset below
-    const char* w;
-    const char* s16;
-    const char* z16;
+    u4 x, w;                    // buffer resources; a stage's k offset is the loads' scalar offset
     uint32_t xoff[C::X_INSTR];  // this lane's byte offsets, fixed for the kernel (see lds_gemm_offsets)
     uint32_t woff[C::W_INSTR];
-    uint32_t poff;              // scales and zeros share it
+    const char* p[C::P_INSTR];  // this lane's scale / zero pair of group 0, and the bytes from a group to the next
+    uint32_t pstep;
+    uint32_t xw, ww, pw;        // this wavefront's first LDS byte of each part of a slot
 };
 
-// Per-lane byte offsets of the direct-to-LDS loads (everything but the stage's k position):
-//   x load i (rows 8 j .. 8 j + 7 of the tile, j = wave X_INSTR + i): lane l takes row rho = 8 j + l / 8
-//     (rows past M read the last row; never stored), 16-byte chunk (l & 7) ^ ((rho >> 1) & 7);
-//   weight load i (row tiles 2 j, 2 j + 1 of the workgroup, j = wave W_INSTR + i): lane l the 16 bytes
-//     l & 31 of the k half of tile 2 j + l / 32's block (tiles past the matrix read its last tile);
-//   params: lane l the values of rows 2 (l & 7), + 1 of the wavefront's tile l / 8 (of NT; NT = 4 repeats).
-template <int MT, int NT, int WM, int WN>
-__device__ __forceinline__ void lds_gemm_offsets(LdsGemmArgs<MT, NT, WM, WN>& a, int M, int K, int G, int m0,
-                                                 int tile0, int tile_last, int wave, int wn, int lane) {
-    using C = LdsGemmCfg<MT, NT, WM, WN>;
+// Per-lane addresses of the direct-to-LDS loads (everything but the stage's k position):
+//   x load j (rows 8 j .. 8 j + 7 of the tile): lane l takes row rho = 8 j + l / 8 (rows past M read the last row;
+//     never stored), 16-byte chunk (l & 7) ^ ((rho >> 1) & 7);
+//   weight load j (row tiles 2 j, 2 j + 1 of the workgroup): lane l the 16 bytes l & 31 of the k half of tile
+//     2 j + l / 32's block (tiles past the matrix read its last tile);
+//   wavefront v issues loads v X_INSTR + i (W_INSTR alike); where those are more than the tile has (a count that does
+//     not divide by the wavefronts), the last wavefronts start earlier and repeat loads of the one before them (the
+//     same bytes to the same place);
+//   params: lane l the values of rows 2 (l & 7), + 1 of one tile: NT <= 4, tile (l / 8) % 4, scales in lanes
+//     0 .. 31 and zeros in 32 .. 63; else tile l / 8 of 8, scales and zeros by a load each. A last tile of 8 rows
+//     (N % 16 == 8) has 16 bytes per group, whose lanes past row 7 read rows 6 and 7 (never stored).
+template <class C>
+__device__ __forceinline__ void lds_gemm_offsets(LdsGemmArgs<C>& a, const h1* scales, const h1* zeros,
+                                                 int M, int N, int K, int G, int m0, int tile0, int tile_last, int wave,
+                                                 int wn, int lane) {
 #pragma unroll
     for (int i = 0; i < C::X_INSTR; ++i) {
-        const int j = wave * C::X_INSTR + i;
+        const int j = min(wave * C::X_INSTR, C::X_LOADS - C::X_INSTR) + i;
         const int rho = 8 * j + (lane >> 3), c = (lane & 7) ^ ((rho >> 1) & 7);
         const int row = min(m0 + rho, M - 1);
         a.xoff[i] = static_cast<uint32_t>(row) * static_cast<uint32_t>(K) * 2u + 16u * c;
     }
 #pragma unroll
     for (int i = 0; i < C::W_INSTR; ++i) {
-        const int j = wave * C::W_INSTR + i;
+        const int j = min(wave * C::W_INSTR, C::W_LOADS - C::W_INSTR) + i;
         const int t = min(tile0 + 2 * j + (lane >> 5), tile_last);
         a.woff[i] = static_cast<uint32_t>(t) * static_cast<uint32_t>(G) * 1024u + 16u * (lane & 31);
     }
-    const int t = min(tile0 + wn * NT + (lane >> 3) % NT, tile_last);
-    a.poff = (static_cast<uint32_t>(t) * 16u * static_cast<uint32_t>(G) + 2u * (lane & 7)) * 2u;
+    const int t = min(tile0 + wn * C::NT + min((lane >> 3) & (C::P_INSTR == 1 ? 3 : 7), C::NT - 1), tile_last);
+    const int rows = tile_rows(t, N);
+    const int64_t off = static_cast<int64_t>(t) * 16 * G + min(2 * (lane & 7), rows - 2);
+    a.pstep = 2u * rows;
+    a.xw = 1024 * min(wave * C::X_INSTR, C::X_LOADS - C::X_INSTR);
+    a.ww = 16 * C::X_U4 + 1024 * min(wave * C::W_INSTR, C::W_LOADS - C::W_INSTR);
+    a.pw = 16 * (C::X_U4 + C::W_U4) + 256 * wave * C::P_INSTR;
+    if constexpr (C::P_INSTR == 1) {
+        a.p[0] = reinterpret_cast<const char*>((lane < 32 ? scales : zeros) + off);
+    } else {
+        a.p[0] = reinterpret_cast<const char*>(scales + off);
+        a.p[1] = reinterpret_cast<const char*>(zeros + off);
+    }
 }
 
-// Issue the direct-to-LDS loads of stage `st` into `slot`. Every wavefront issues exactly LOADS
-// instructions, so each can wait for a stage with one vmcnt. Stage st = (group g, k half h) moves the
-// bases only: x by (128 g + 64 h) halves, the weights by block g and half h (g * 1024 + h * 512 bytes),
-// the scales and zeros by group g (16 g halves of every tile).
-template <int MT, int NT, int WM, int WN>
-__device__ __forceinline__ void issue_stage(uint32_t slot, const LdsGemmArgs<MT, NT, WM, WN>& a, int st, int wave) {
-    using C = LdsGemmCfg<MT, NT, WM, WN>;
-    const int g = st >> 1, h = st & 1;
-    const char* xb = a.x + (256 * g + 128 * h);
-#pragma unroll
-    for (int i = 0; i < C::X_INSTR; ++i) lds_dma<16>(xb, a.xoff[i], slot + 16 * 64 * (wave * C::X_INSTR + i));
-    const char* wb = a.w + (1024 * g + 512 * h);
-#pragma unroll
-    for (int i = 0; i < C::W_INSTR; ++i)
-        lds_dma<16>(wb, a.woff[i], slot + 16 * (C::X_U4 + 64 * (wave * C::W_INSTR + i)));
-    const uint32_t pslot = slot + 16 * (C::X_U4 + C::W_U4 + wave * 32);
-    lds_dma<4>(a.s16 + 32 * g, a.poff, pslot);         // scales [8 tiles][16 rows]
-    lds_dma<4>(a.z16 + 32 * g, a.poff, pslot + 256);   // zeros, the same order
+// Direct-to-LDS load I (of X_INSTR + W_INSTR, then P_INSTR at even stages) of stage `st` into the slot at LDS byte
+// address `slot`. Every wavefront issues the same number per stage, so each can wait for a stage with one vmcnt.
+// Stage st = (group g = st / 2, k half st & 1) moves the scalar offset only: x by 64 st halves, the weights by block g
+// and half (512 st bytes), the scales and zeros by group g (pg; past the last group its own again).
+template <int I, class C>
+__device__ __forceinline__ void issue_load(uint32_t slot, const LdsGemmArgs<C>& a, const u4& xr, const u4& wr,
+                                           int st, int pg) {
+    if constexpr (I < C::X_INSTR)
+        lds_dma16<1024 * I>(xr, a.xoff[I], 128u * st, slot + a.xw);
+    else if constexpr (I < C::XW)
+        lds_dma16<1024 * (I - C::X_INSTR)>(wr, a.woff[I - C::X_INSTR], 512u * st, slot + a.ww);
+    else
+        lds_dma4<256 * (I - C::XW)>(a.p[I - C::XW] + static_cast<uint64_t>(static_cast<uint32_t>(pg)) * a.pstep, slot + a.pw);
 }
 
-// One stage's math from `slot`: two substeps of NT x MT MFMAs.
-template <int MT, int NT, int WM, int WN>
-__device__ __forceinline__ void compute_stage(const u4* slot, f4 (&acc)[NT][MT], int wave, int wm, int wn, int lane,
-                                              uint32_t magic) {
-    using C = LdsGemmCfg<MT, NT, WM, WN>;
-    // One wavefront along M: let the scheduler interleave the MFMAs with the LDS reads and the dequant
-    // (LLVM's IGroupLP strategy 0). Measured on the 128 x 256 tile at M = 2048 / 4096: gate_up 364.6 ->
-    // 360.1 / 706.3 -> 696.7 us, down 204.1 -> 200.8 / 336.3 -> 334.4 us; on the WM = 2 tiles it was
-    // slower, so they keep the default schedule. The MFMA order per accumulator is unchanged.
-    if constexpr (WM == 1) __builtin_amdgcn_iglp_opt(0);
-    const int r = lane & 15, q = lane >> 4;
-    const u4* xs = slot;
-    const u4* ws = slot + C::X_U4;
-    const uint16_t* ps = reinterpret_cast<const uint16_t*>(slot + C::X_U4 + C::W_U4 + wave * 32);  // [2][8][16]
-    // lane (q, r) needs words s = q & 1 and 2 + (q & 1) of (kb = 2 h + (q >> 1), r): one ds_read2_b32
-    uint32_t wv[NT][2];
-    GroupQ pq[NT];
+// The loads of LOADS per stage that step k of S issues (evenly spread), from load I on.
+template <int I, int LOADS, int S, class C>
+__device__ __forceinline__ void issue_loads_at(int k, uint32_t slot, const LdsGemmArgs<C>& a, const u4& xr,
+                                               const u4& wr, int st, int pg) {
+    if constexpr (I < LOADS) {
+        if ((2 * I + 1) * S / (2 * LOADS) == k) issue_load<I>(slot, a, xr, wr, st, pg);
+        issue_loads_at<I + 1, LOADS, S>(k, slot, a, xr, wr, st, pg);
+    }
+}
+
+// Registers of the software pipeline: the B fragments of the current and the next 32-k substep, the current and next
+// half group's weight words (WK = 1: one 8-byte pair per tile, both substeps; WK = 2: the wavefront's one), the
+// group's dequantization constants.
+template <class C>
+struct LdsGemmRegs {
+    h8 xb[2][C::MT];
+    uint32_t wv[2][C::NT][3 - C::WK];
+    GroupQ pq[C::NT];
+    uint32_t ps[C::NT], pz[C::NT];
+    h8 a;  // the dequantized A fragment of the next (substep, tile)
+};
+
+template <class C>
+__device__ __forceinline__ void read_words(uint32_t (&w)[3 - C::WK], const char* p) {
+    if constexpr (C::WK == 1) {
+        const u2 v = *reinterpret_cast<const u2*>(p);
+        w[0] = v.x, w[1] = v.y;
+    } else {
+        w[0] = *reinterpret_cast<const uint32_t*>(p);
+    }
+}
+
+// One 32-k substep of a half group of parity PAR (0: k half 0), B fragments in set CUR and words J of set PAR: NT
+// steps of MT MFMAs, beside which the next substep's B fragments are read from `nxt` (front-loaded over the first
+// steps) and the next step's A fragment is dequantized. LAST, the wavefront's last substep of its half group: the
+// words (and at PAR = 1 the scales and zeros) of the next half group are read too and LOADS loads of stage `st`
+// issued into slot address `dma`. All of it sits between the MFMAs, at most a few instructions behind each, because
+// a wavefront issues in order: side work in a block of its own leaves the matrix core idle after 16 cycles.
+template <class C, int PAR, int CUR, int J, bool LAST, int LOADS>
+__device__ __forceinline__ void substep(LdsGemmRegs<C>& v, f4 (&acc)[C::NT][C::MT], const u4* nxt, int xl, int wl, int pl,
+                                        uint32_t dma, const LdsGemmArgs<C>& a, const u4& xr, const u4& wr, int st, int pg,
+                                        uint32_t magic) {
+    constexpr int MT = C::MT, NT = C::NT;
+    constexpr int S = NT * MT;  // steps: one MFMA and the side work that issues while it runs
+    const char* nb = reinterpret_cast<const char*>(nxt);
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
-        const uint32_t* wp = reinterpret_cast<const uint32_t*>(ws + (wn * NT + t) * 32 + (q >> 1) * 16 + r) + (q & 1);
-        wv[t][0] = wp[0];
-        wv[t][1] = wp[2];
-        pq[t] = group_q(as_h1(ps[t * 16 + r]), as_h1(ps[128 + t * 16 + r]));
-    }
-    // both substeps' B fragments are read up front, so the second substep's LDS latency hides under the
-    // first substep's MFMAs
-    h8 xb[2][MT];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-        const int c = 4 * (q >> 1) + 2 * j + (q & 1);
+        const h8 at = v.a;
+        // the next step's tile: its word and constants
+        const bool same = t + 1 < NT;
+        const int tn = same ? t + 1 : 0;
+        h2 d[4];
 #pragma unroll
         for (int b = 0; b < MT; ++b) {
-            const int rho = wm * 16 * MT + 16 * b + r;
-            xb[j][b] = bitcast<h8>(xs[rho * 8 + (c ^ ((rho >> 1) & 7))]);
+            const int k = t * MT + b;
+            if (b == 0)
+                mfma_acc<true>(acc[t][b], at, v.xb[CUR][b]);
+            else
+                mfma_acc<false>(acc[t][b], at, v.xb[CUR][b]);
+            if (LAST && k < NT) read_words<C>(v.wv[1 - PAR][k], nb + wl + 512 * k);  // the next half group's words,
+            if (LAST && PAR == 1 && k >= 1 && k <= NT) {                             // then its scales and zeros
+                const uint16_t* ps = reinterpret_cast<const uint16_t*>(nb + pl);
+                v.ps[k - 1] = ps[16 * (k - 1)], v.pz[k - 1] = ps[(NT <= 4 ? 64 : 128) + 16 * (k - 1)];
+            }
+#pragma unroll
+            for (int i = 0; i < MT; ++i)  // B fragment i in the first half of the steps
+                if (i * S / (2 * MT) == k) v.xb[1 - CUR][i] = bitcast<h8>(*(reinterpret_cast<const u4*>(nb + xl) + 128 * i));
+            // tile t's constants of the next group, once its words of this one are done with
+            if (LAST && PAR == 1 && b == (MT > 4 ? MT / 2 : MT - 1) && same) v.pq[t] = group_q(as_h1(v.ps[t]), as_h1(v.pz[t]));
+            if (LAST && PAR == 1 && b == 0 && !same) v.pq[NT - 1] = group_q(as_h1(v.ps[NT - 1]), as_h1(v.pz[NT - 1]));
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if ((2 * i + 1) * MT / 8 == b) {
+                    const uint32_t word = same ? v.wv[PAR][tn][J] : LAST ? v.wv[1 - PAR][0][0] : v.wv[PAR][0][C::WK == 1 ? 1 : 0];
+                    d[i] = dequant_pair(word, i, v.pq[tn], magic);
+                }
+            issue_loads_at<0, LOADS, S>(k, dma, a, xr, wr, st, pg);
+            TW4_STEP_FENCE;
         }
-    }
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const h8 a = dequant_word(wv[t][j], pq[t], magic);
-#pragma unroll
-            for (int b = 0; b < MT; ++b) acc[t][b] = mfma16x16x32(a, xb[j][b], acc[t][b]);
-        }
+        v.a = h8{d[0].x, d[0].y, d[1].x, d[1].y, d[2].x, d[2].y, d[3].x, d[3].y};
     }
 }
 
-// One step of a ring of R slots with compile-time slot S: wait for stage i (leaving the later stages
-// already issued in flight: up to R - 2 of them), barrier, issue stage i + R - 1 into the slot
-// (S + R - 1) % R that stage i - 1 used, compute stage i from slot S.
-template <int S, int R, int MT, int NT, int WM, int WN>
-__device__ __forceinline__ void ring_step(const u4* ring, uint32_t ring_addr, const LdsGemmArgs<MT, NT, WM, WN>& a,
-                                          int i, int nst, int st0, f4 (&acc)[NT][MT], int wave, int wm, int wn,
-                                          int lane, uint32_t magic) {
-    using C = LdsGemmCfg<MT, NT, WM, WN>;
-    const int ahead = min(nst - 1 - i, R - 2);  // stages after i already in flight
-    if constexpr (R == 4) {
-        if (ahead >= 2)
-            wait_vmcnt<2 * C::LOADS>();
-        else if (ahead == 1)
-            wait_vmcnt<C::LOADS>();
-        else
-            wait_vmcnt<0>();
-    } else {
-        if (ahead >= 1)
-            wait_vmcnt<C::LOADS>();
-        else
-            wait_vmcnt<0>();
+// Half group i (parity PAR) from ring slot `slot`, which then moves to the next one. WK = 1: substep 0 reads the
+// second substep's fragments from the slot. Then the wavefront waits for its own loads of stage i + 1 (the R - 2
+// stages after it stay in flight) and for its LDS reads of stage i, and the workgroup meets: stage i + 1 is in LDS
+// and nobody reads stage i any more, so its slot takes the loads of stage i + R beside the last substep's math,
+// which reads stage i + 1. A stage past the end is issued with empty resources. WK = 2: each wavefront has one of
+// the two substeps, read a whole half group ahead.
+template <class C, int PAR>
+__device__ __forceinline__ void half_step(LdsGemmRegs<C>& v, f4 (&acc)[C::NT][C::MT], const u4* ring, uint32_t ring_addr,
+                                          int& slot, int i, int nst, int st0, int xl0, int xl1, int wl, int pl,
+                                          const LdsGemmArgs<C>& a, int glast, uint32_t magic) {
+    constexpr int R = C::R;
+    const u4* cur = ring + slot * C::SLOT_U4;
+    const uint32_t cur_addr = ring_addr + 16 * slot * C::SLOT_U4;
+    slot = slot + 1 == R ? 0 : slot + 1;
+    const u4* nxt = ring + slot * C::SLOT_U4;
+    if constexpr (C::WK == 1) {
+        const u4 none{};
+        substep<C, PAR, 0, 0, false, 0>(v, acc, cur, xl1, wl, pl, 0, a, none, none, 0, 0, magic);
     }
+    // loads of stages i + 2 .. i + R - 1: R - 2 stages, the first of this one's parity, params with the even ones
+    constexpr int AHEAD = (R - 2) * C::XW + (R - 2 + (PAR == 0 ? 1 : 0)) / 2 * C::P_INSTR;
+    constexpr int LOADS = C::XW + ((PAR + R) % 2 == 0 ? C::P_INSTR : 0);
+    wait_stage<AHEAD>();
     ring_barrier();
-    if (i + R - 1 < nst)
-        issue_stage<MT, NT, WM, WN>(ring_addr + 16 * ((S + R - 1) % R) * C::SLOT_U4, a, st0 + i + R - 1, wave);
-    compute_stage<MT, NT, WM, WN>(ring + S * C::SLOT_U4, acc, wave, wm, wn, lane, magic);
-    __builtin_amdgcn_sched_barrier(0);  // one stage's registers at a time: no scheduling across steps
+    const int st = st0 + i + R;
+    u4 xr = a.x, wr = a.w;
+    xr.z = wr.z = __builtin_amdgcn_readfirstlane(i + R < nst ? 0xFFFFFFFFu : 0u);
+    substep<C, PAR, C::WK == 1 ? 1 : PAR, C::WK == 1 ? 1 : 0, true, LOADS>(v, acc, nxt, xl0, wl, pl, cur_addr, a, xr, wr, st,
+                                                                        min(st >> 1, glast), magic);
 }
 
-template <int MT, int NT, int WM, int WN, int R>
-__global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_eu(LdsGemmCfg<MT, NT, WM, WN>::MIN_WAVES_PER_SIMD))) gemm_lds_kernel(const h1* __restrict__ x, const u4* __restrict__ w,
-                                                               const h1* __restrict__ scales,
-                                                               const h1* __restrict__ zeros, h1* __restrict__ y,
-                                                               float* __restrict__ ws, int* __restrict__ locks, int M,
-                                                               int N, int K, int mb, int nb, int splits, int act) {
-    using C = LdsGemmCfg<MT, NT, WM, WN>;
-    static_assert(R == 3 || R == 4, "ring of 3 or 4 slots");
-    __shared__ u4 ring[R * C::SLOT_U4];
+template <class C>
+__global__ void __launch_bounds__(C::THREADS) __attribute__((amdgpu_waves_per_eu(C::MIN_WAVES_PER_SIMD)))
+gemm_lds_kernel(const h1* __restrict__ x, const u4* __restrict__ w, const h1* __restrict__ scales,
+                const h1* __restrict__ zeros, h1* __restrict__ y, float* __restrict__ ws, int* __restrict__ locks,
+                int M, int N, int K, int mb, int nb, int splits, int act) {
+    __shared__ u4 ring[C::R * C::SLOT_U4];
     __shared__ int last_flag;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wn = wave % WN, wm = wave / WN;
-    const int G = K >> 7, tiles_n = (N + 15) >> 4, stages = 2 * G;
+    constexpr int MT = C::MT, NT = C::NT, R = C::R;
+    const int wn = wave % C::WN, wm = wave / C::WN % C::WM, wk = wave / (C::WN * C::WM);
+    const int G = K >> 7, tiles_n = (N + 15) >> 4;
 
     // work unit -> (tile, split); tiles in bands of 8 token blocks, each XCD a contiguous range
     const int unit = xcd_remap(blockIdx.x, gridDim.x);
     const int tile = unit / splits, split = unit - tile * splits;
     const int band = tile / (8 * nb), band_rows = min(mb - band * 8, 8), rin = tile - band * 8 * nb;
     const int mblk = band * 8 + rin % band_rows, nblk = rin / band_rows;
-    const int st0 = static_cast<int>(static_cast<int64_t>(split) * stages / splits);
-    const int nst = static_cast<int>(static_cast<int64_t>(split + 1) * stages / splits) - st0;
+    // whole quant groups per split; a split past the groups has none and contributes zeros
+    const int g0 = static_cast<int>(static_cast<int64_t>(split) * G / splits);
+    const int nst = 2 * (static_cast<int>(static_cast<int64_t>(split + 1) * G / splits) - g0);
+    const int st0 = 2 * g0;
 
     const int m0 = mblk * C::BM, tile0 = nblk * (C::BN / 16);
-    LdsGemmArgs<MT, NT, WM, WN> a;
-    a.x = reinterpret_cast<const char*>(x);
-    a.w = reinterpret_cast<const char*>(w);
-    a.s16 = reinterpret_cast<const char*>(scales);
-    a.z16 = reinterpret_cast<const char*>(zeros);
-    lds_gemm_offsets<MT, NT, WM, WN>(a, M, K, G, m0, tile0, tiles_n - 1, wave, wn, lane);
+    LdsGemmArgs<C> a;
+    a.x = lds_rsrc(x);
+    a.w = lds_rsrc(w);
+    lds_gemm_offsets<C>(a, scales, zeros, M, N, K, G, m0, tile0, tiles_n - 1, wave, wn, lane);
 
     const uint32_t magic = magic_reg();
     f4 acc[NT][MT];
@@ -265,37 +316,87 @@ __global__ void __launch_bounds__(64 * WM * WN) __attribute__((amdgpu_waves_per_
 #pragma unroll
         for (int b = 0; b < MT; ++b) acc[t][b] = f4{0.0f, 0.0f, 0.0f, 0.0f};
 
-    // the ring's LDS byte address, taken once from the array itself (the direct-to-LDS loads take it in M0)
-    const uint32_t ring_addr = static_cast<uint32_t>(reinterpret_cast<size_t>((lds_void*)ring));
+    if (nst > 0) {
+        // the ring's LDS byte address, taken once from the array itself (the direct-to-LDS loads take it in M0)
+        const uint32_t ring_addr = static_cast<uint32_t>(reinterpret_cast<size_t>((lds_void*)ring));
+        const int r = lane & 15, q = lane >> 4;
+        // byte offsets inside a slot: this lane's 16-byte chunk of token row r at the wavefront's first substep (the
+        // other one: ^ 16), its words of the wavefront's first tile, the row's scale of that tile
+        const int c0 = 4 * (q >> 1) + 2 * (q & 1);
+        const int xl0 = (wm * 16 * MT + r) * 128 + 16 * ((c0 + wk) ^ ((r >> 1) & 7)), xl1 = xl0 ^ 16;
+        const int wl = 16 * C::X_U4 + wn * NT * 512 + ((q >> 1) * 16 + r) * 16 + 8 * (q & 1) + 4 * wk;
+        const int pl = 16 * (C::X_U4 + C::W_U4) + 256 * wave * C::P_INSTR + 2 * r;
 #pragma unroll
-    for (int p = 0; p < R - 1; ++p)
-        if (p < nst) issue_stage<MT, NT, WM, WN>(ring_addr + 16 * p * C::SLOT_U4, a, st0 + p, wave);
-    for (int i = 0; i < nst; i += R) {
-        ring_step<0, R>(ring, ring_addr, a, i, nst, st0, acc, wave, wm, wn, lane, magic);
-        if (i + 1 < nst) ring_step<1, R>(ring, ring_addr, a, i + 1, nst, st0, acc, wave, wm, wn, lane, magic);
-        if (i + 2 < nst) ring_step<2, R>(ring, ring_addr, a, i + 2, nst, st0, acc, wave, wm, wn, lane, magic);
-        if constexpr (R == 4)
-            if (i + 3 < nst) ring_step<3, R>(ring, ring_addr, a, i + 3, nst, st0, acc, wave, wm, wn, lane, magic);
+        for (int p = 0; p < R; ++p) {
+            u4 xr = a.x, wr = a.w;
+            xr.z = wr.z = __builtin_amdgcn_readfirstlane(p < nst ? 0xFFFFFFFFu : 0u);
+            const uint32_t sa = ring_addr + 16 * p * C::SLOT_U4;
+            if (p & 1)
+                issue_loads_at<0, C::XW, 1>(0, sa, a, xr, wr, st0 + p, 0);
+            else
+                issue_loads_at<0, C::XW + C::P_INSTR, 1>(0, sa, a, xr, wr, st0 + p, min(g0 + (p >> 1), G - 1));
+        }
+        wait_stage<(R - 1) * C::XW + (R - 1) / 2 * C::P_INSTR>();  // stages 1 .. R - 1 may be in flight
+        ring_barrier();
+        LdsGemmRegs<C> v;
+        {
+            const char* s0 = reinterpret_cast<const char*>(ring);
+            const uint16_t* ps = reinterpret_cast<const uint16_t*>(s0 + pl);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) {
+                read_words<C>(v.wv[0][t], s0 + wl + 512 * t);
+                v.pq[t] = group_q(as_h1(ps[16 * t]), as_h1(ps[(NT <= 4 ? 64 : 128) + 16 * t]));
+            }
+#pragma unroll
+            for (int b = 0; b < MT; ++b) v.xb[0][b] = bitcast<h8>(*(reinterpret_cast<const u4*>(s0 + xl0) + 128 * b));
+            v.a = dequant_word(v.wv[0][0][0], v.pq[0], magic);
+        }
+        int slot = 0, i = 0;
+        for (; i < nst; i += 2) {
+            half_step<C, 0>(v, acc, ring, ring_addr, slot, i, nst, st0, xl0, xl1, wl, pl, a, G - 1, magic);
+            half_step<C, 1>(v, acc, ring, ring_addr, slot, i + 1, nst, st0, xl0, xl1, wl, pl, a, G - 1, magic);
+        }
+        mfma_settle<NT, MT>(acc);
+        wait_stage<0>();  // the empty loads past the end still write their slots
     }
 
-    finish_unit<MT, NT, WM * WN>(acc, true, wave, lane, tid, splits, tile, unit, ws, locks, last_flag, y, M, N,
+    if constexpr (C::WK == 2) {  // the K halves' sums: the ring is free (every load has landed, every read is done)
+        __syncthreads();
+        f4* red = reinterpret_cast<f4*>(ring) + (wm * C::WN + wn) * NT * MT * 64 + lane;
+        if (wk == 1) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int b = 0; b < MT; ++b) red[(t * MT + b) * 64] = acc[t][b];
+        }
+        __syncthreads();
+        if (wk == 0) {
+#pragma unroll
+            for (int t = 0; t < NT; ++t)
+#pragma unroll
+                for (int b = 0; b < MT; ++b) acc[t][b] += red[(t * MT + b) * 64];
+        }
+    }
+    finish_unit<MT, NT, C::WM * C::WN>(acc, wk == 0, wm * C::WN + wn, lane, tid, splits, tile, unit, ws, locks, last_flag, y, M, N,
                                  m0 + wm * 16 * MT, tile0 + wn * NT, tiles_n, act);
 }
 
-// Compiled configurations (MT, NT, WM, WN, ring slots).
-#define TW4_LDS_GEMM_CONFIGS(X) X(8, 4, 2, 4, 3) X(16, 4, 1, 4, 3) X(4, 4, 2, 4, 3) X(8, 4, 2, 2, 3) X(8, 8, 1, 4, 4) X(8, 4, 1, 4, 3)
+// Compiled configurations (MT, NT, WM, WN, WK, ring slots): tw4_gemm's stages-3 ones, and the others of tw4_gemm_tiled.
+#define TW4_LDS_GEMM_CONFIGS(X) X(8, 4, 2, 4, 1, 3) X(16, 4, 1, 4, 1, 3) X(4, 4, 2, 4, 1, 3) X(8, 4, 2, 2, 1, 3) \
+    X(8, 8, 1, 4, 1, 4) X(8, 4, 1, 4, 1, 3)
+#define TW4_TILED_GEMM_CONFIGS(X) X(8, 6, 2, 2, 1, 3) X(8, 6, 1, 2, 2, 4) X(8, 4, 1, 2, 2, 4) X(8, 3, 1, 2, 2, 4) \
+    X(8, 2, 1, 2, 2, 4) X(5, 4, 1, 2, 2, 4) X(5, 3, 1, 2, 2, 4) X(5, 2, 1, 2, 2, 4) X(4, 3, 1, 2, 2, 4) \
+    X(4, 2, 1, 2, 2, 4) X(3, 3, 1, 2, 2, 4) X(3, 2, 1, 2, 2, 4) X(2, 3, 1, 2, 2, 4) X(2, 2, 1, 2, 2, 4)
 
-template <int MT, int NT, int WM, int WN, int R>
+template <class C>
 int lds_gemm_launch(const h1* x, const u4* w, const h1* s, const h1* z, h1* y, float* ws, int* locks,
                     int64_t ws_floats, int64_t n_locks, int M, int N, int K, int splits, int cus, int act,
                     hipStream_t stream) {
-    using C = LdsGemmCfg<MT, NT, WM, WN>;
-    TW4_REQUIRE(N % 16 == 0, TW4_EINVAL, "gemm (stages 3): N %% 16 == 0 (N = %d)", N);
     // the loads' per-lane byte offsets are 32-bit: x (M K 2 bytes) and the weights (N K / 2 bytes)
     TW4_REQUIRE(static_cast<int64_t>(M) * K < (1LL << 31) && static_cast<int64_t>(N) * K < (1LL << 33), TW4_EINVAL,
-                "gemm (stages 3): M K < 2^31 and N K < 2^33 (M %d, N %d, K %d)", M, N, K);
-    TW4_REQUIRE(reinterpret_cast<uintptr_t>(s) % 16 == 0 && reinterpret_cast<uintptr_t>(z) % 16 == 0, TW4_EINVAL,
-                "gemm (stages 3): scales and zeros must be 16-byte aligned");
+                "gemm (both tiles in LDS): M K < 2^31 and N K < 2^33 (M %d, N %d, K %d)", M, N, K);
+    TW4_REQUIRE(reinterpret_cast<uintptr_t>(s) % 4 == 0 && reinterpret_cast<uintptr_t>(z) % 4 == 0, TW4_EINVAL,
+                "gemm (both tiles in LDS): scales and zeros must be 4-byte aligned");
     const int G = K >> 7, stages = 2 * G;
     const int mb = (M + C::BM - 1) / C::BM, nb = (N + C::BN - 1) / C::BN;
     const int64_t tiles64 = static_cast<int64_t>(mb) * nb;
@@ -317,9 +418,9 @@ int lds_gemm_launch(const h1* x, const u4* w, const h1* s, const h1* z, h1* y, f
     }
     const int64_t blocks = static_cast<int64_t>(tiles) * sp;
     TW4_REQUIRE(blocks < (1LL << 31), TW4_EINVAL, "gemm: grid too large");
-    gemm_lds_kernel<MT, NT, WM, WN, R><<<static_cast<unsigned>(blocks), C::THREADS, 0, stream>>>(
+    gemm_lds_kernel<C><<<static_cast<unsigned>(blocks), C::THREADS, 0, stream>>>(
         x, w, s, z, y, ws, locks, M, N, K, mb, nb, sp, act);
-    TW4_LAUNCH_CHECK("gemm (stages 3): launch");
+    TW4_LAUNCH_CHECK("gemm (both tiles in LDS): launch");
     return TW4_OK;
 }
 
@@ -332,16 +433,19 @@ int tw4_gemm_lds_dispatch(const uint16_t* x, const int32_t* packed, const uint16
                           uint16_t* y, float* ws, int32_t* locks, int64_t ws_floats, int64_t n_locks, int M, int N,
                           int K, int mt, int nt, int warps_n, int warps_m, int splits, int cus, int act,
                           void* stream) {
+    TW4_REQUIRE(N % 16 == 0, TW4_EINVAL, "gemm (stages 3): N %% 16 == 0 (N = %d)", N);
+    TW4_REQUIRE(reinterpret_cast<uintptr_t>(scales) % 16 == 0 && reinterpret_cast<uintptr_t>(zeros) % 16 == 0, TW4_EINVAL,
+                "gemm (stages 3): scales and zeros must be 16-byte aligned");
     auto xp = reinterpret_cast<const h1*>(x);
     auto wp = reinterpret_cast<const u4*>(packed);
     auto sp = reinterpret_cast<const h1*>(scales);
     auto zp = reinterpret_cast<const h1*>(zeros);
     auto yp = reinterpret_cast<h1*>(y);
     auto st = static_cast<hipStream_t>(stream);
-#define TW4_LDS_CASE(MT, NT, WM, WN, R)                                                                           \
-    if (mt == MT && nt == NT && warps_m == WM && warps_n == WN)                                                      \
-        return lds_gemm_launch<MT, NT, WM, WN, R>(xp, wp, sp, zp, yp, ws, locks, ws_floats, n_locks, M, N, K, splits, \
-                                                  cus, act, st);
+#define TW4_LDS_CASE(MT, NT, WM, WN, WK, R)                                                                            \
+    if (mt == MT && nt == NT && warps_m == WM && warps_n == WN)                                                        \
+        return lds_gemm_launch<LdsGemmCfg<MT, NT, WM, WN, WK, R>>(xp, wp, sp, zp, yp, ws, locks, ws_floats, n_locks, M,\
+                                                                  N, K, splits, cus, act, st);
     TW4_LDS_GEMM_CONFIGS(TW4_LDS_CASE)
 #undef TW4_LDS_CASE
     tw4host::set_error("gemm: unsupported stages-3 config mt / nt / warps_n / warps_m %d / %d / %d / %d", mt, nt,
@@ -349,9 +453,32 @@ int tw4_gemm_lds_dispatch(const uint16_t* x, const int32_t* packed, const uint16
     return TW4_ECONFIG;
 }
 
+// Called by tw4_gemm_tiled.
+int tw4_gemm_tiled_dispatch(const uint16_t* x, const int32_t* packed, const uint16_t* scales, const uint16_t* zeros,
+                            uint16_t* y, float* ws, int32_t* locks, int64_t ws_floats, int64_t n_locks, int M, int N,
+                            int K, int mt, int nt, int warps_n, int warps_m, int warps_k, int ring, int splits, int cus,
+                            int act, void* stream) {
+    auto xp = reinterpret_cast<const h1*>(x);
+    auto wp = reinterpret_cast<const u4*>(packed);
+    auto sp = reinterpret_cast<const h1*>(scales);
+    auto zp = reinterpret_cast<const h1*>(zeros);
+    auto yp = reinterpret_cast<h1*>(y);
+    auto st = static_cast<hipStream_t>(stream);
+#define TW4_LDS_CASE(MT, NT, WM, WN, WK, R)                                                                            \
+    if (mt == MT && nt == NT && warps_m == WM && warps_n == WN && warps_k == WK && ring == R)                          \
+        return lds_gemm_launch<LdsGemmCfg<MT, NT, WM, WN, WK, R>>(xp, wp, sp, zp, yp, ws, locks, ws_floats, n_locks, M,\
+                                                                  N, K, splits, cus, act, st);
+    TW4_LDS_GEMM_CONFIGS(TW4_LDS_CASE)
+    TW4_TILED_GEMM_CONFIGS(TW4_LDS_CASE)
+#undef TW4_LDS_CASE
+    tw4host::set_error("gemm_tiled: unsupported mt / nt / warps_n / warps_m / warps_k / ring %d / %d / %d / %d / %d / %d", mt,
+                       nt, warps_n, warps_m, warps_k, ring);
+    return TW4_ECONFIG;
+}
+
 int tw4_gemm_lds_configs(int* out, int max_configs, int start) {
     int n = 0;
-#define TW4_LDS_LIST(MT, NT, WM, WN, R)              \
+#define TW4_LDS_LIST(MT, NT, WM, WN, WK, R)              \
     if (out && start + n < max_configs) {            \
         out[5 * (start + n)] = MT;                   \
         out[5 * (start + n) + 1] = NT;               \
@@ -361,6 +488,24 @@ int tw4_gemm_lds_configs(int* out, int max_configs, int start) {
     }                                                \
     ++n;
     TW4_LDS_GEMM_CONFIGS(TW4_LDS_LIST)
+#undef TW4_LDS_LIST
+    return n;
+}
+
+extern "C" int tw4_gemm_tiled_configs(int* out, int max_configs) {
+    int n = 0;
+#define TW4_LDS_LIST(MT, NT, WM, WN, WK, R)    \
+    if (out && n < max_configs) {          \
+        out[6 * n] = MT;                   \
+        out[6 * n + 1] = NT;               \
+        out[6 * n + 2] = WN;               \
+        out[6 * n + 3] = WM;               \
+        out[6 * n + 4] = WK;               \
+        out[6 * n + 5] = R;                \
+    }                                      \
+    ++n;
+    TW4_LDS_GEMM_CONFIGS(TW4_LDS_LIST)
+    TW4_TILED_GEMM_CONFIGS(TW4_LDS_LIST)
 #undef TW4_LDS_LIST
     return n;
 }

@@ -39,7 +39,7 @@ import torch
 import torch.nn.functional as F
 from torch import nn
 
-from tandem_amd.layers import w4_hip
+from tandem_amd.layers import w4_hip, w4_plan
 from tandem_amd.layers.w4_tables import GFX950_DECODE, GFX950_GEMM
 
 # Nibble of an AutoAWQ word that holds feature j = 0..7 of its 8: the packer writes features
@@ -167,20 +167,16 @@ W4_KERNELS: dict[str, dict[tuple, W4Kernel]] = {
     GFX950: GFX950_DECODE,
 }
 
-# GEMM for M > 16 per GPU and (N, K) / (N, K, "silu"): ((m_max, config), ...) by increasing m_max;
-# M past the last m_max uses the last entry. config = (MT, NT, WARPS_N, WARPS_K, STAGES, SPLITS) of
-# w4_gemm (BM = 16 MT tokens, each wavefront 16 NT rows, WARPS_N x WARPS_K wavefronts, STAGES-deep
-# LDS ring, SPLITS: split-K of every tile, or 0: of the last, partial wave of tiles only), or
-# ("mma", warps_k, unroll, ntile): the streaming matrix-core kernel of the decode path, whose 16-token
-# batch tiles cover M <= 64 (bandwidth-bound batches), or None: dequantize to float16 +
-# torch.matmul. Shapes without an entry use DEFAULT_GEMM, which stops at M = 1024 like the measured
-# gfx950 ladders before the GEMM with both tiles staged through LDS (stages 3): on the Qwen3-8B shapes
-# that GEMM carries the fused path to M = 2048, and past it the dequantize + hipBLASLt pair wins (by
-# ~20 % at M = 4096), since the one-off dequant is small next to the product there.
+# M > 16: measured ladders per GPU and (N, K) / (N, K, "silu"), ((m_max, config), ...) by increasing m_max. config =
+# (MT, NT, WARPS_N, WARPS_K, STAGES, SPLITS) of w4_gemm, ("mma", warps_k, unroll, ntile): the streaming matrix-core kernel
+# of the decode path, whose 16-token batch tiles cover M <= 64, ("tiled", MT, NT, WARPS_N, WARPS_M, WARPS_K, RING, SPLITS)
+# of w4_gemm_tiled, or None: dequantize to float16 + torch.matmul. Past a ladder's last m_max, and for shapes without
+# one, w4_plan.choose picks the kernel from the sizes (the built-in ladders end at M = 64: past it the rule's choice is
+# as fast as the measured rungs were, and faster wherever w4_gemm_tiled is). DEFAULT_GEMM is the ladder of shapes
+# without an entry: no rung.
 # TANDEM_W4_GEMM=0: always dequantize + torch.matmul (python/tandem/layers/awq.py:163-186).
 W4Gemm = tuple
-DEFAULT_GEMM: tuple[tuple[int, W4Gemm | None], ...] = (
-    (64, ("mma", 8, 1, 1)), (1024, (4, 2, 4, 1, 2, 0)), (1 << 30, None))
+DEFAULT_GEMM: tuple[tuple[int, W4Gemm | None], ...] = ()
 W4_GEMM_KERNELS: dict[str, dict[tuple, tuple[tuple[int, W4Gemm | None], ...]]] = {
     MI355X: GFX950_GEMM,
     GFX950: GFX950_GEMM,
@@ -226,6 +222,12 @@ def _table(tables: dict, device_name: str | None, device: torch.device) -> dict:
     return {}
 
 
+def _plain(x: torch.Tensor) -> bool:
+    """No gradient is asked of x and no transform (vmap, jvp) wraps it: a call that dequantize + F.linear would have to
+    carry through autograd or a transform must not go to a kernel that sees a data pointer only."""
+    return not (x.requires_grad and torch.is_grad_enabled()) and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+
+
 # Chunks (16 bytes of x) one wavefront stages in one batch: 64 lanes x 2 (kXB in tw4_decode.hip).
 FUSED_NORM_CHUNKS = 128
 
@@ -257,6 +259,7 @@ class W4Linear(nn.Module):
         self.register_buffer("scales", torch.empty(in_features // group, out_features, dtype=torch.float16))
         self.kernels: dict[tuple, W4Kernel] = {}
         self.gemm_kernels: dict[tuple, tuple[tuple[int, W4Gemm | None], ...]] = {}
+        self.cus = 256  # of the layer's GPU, for the rule (finalize)
 
     def enable_silu_mul(self) -> bool:
         if not self.awq_layout or self.out_features % 16:
@@ -275,9 +278,11 @@ class W4Linear(nn.Module):
         self.awq_layout = False
         self.kernels = _table(W4_KERNELS, device_name, packed.device)
         self.gemm_kernels = _table(W4_GEMM_KERNELS, device_name, packed.device)
+        self.cus = torch.cuda.get_device_properties(packed.device).multi_processor_count
         # device set-up and the split-K workspace now, not inside graph capture
         if w4_hip.load() is not None:
             w4_hip.workspace(packed.device)
+            w4_hip.stream_workspace(packed.device)
 
     def _dense(self, x: torch.Tensor) -> torch.Tensor:
         """HIP dequantize (gate_up: back in [gate | up] row order) + torch.matmul, and the same
@@ -289,8 +294,23 @@ class W4Linear(nn.Module):
         return silu_and_mul(y) if self.silu_mul else y
 
     def _gemm(self, ext, x: torch.Tensor, cfg) -> torch.Tensor:
-        buf, locks = w4_hip.workspace(x.device)
-        return ext.w4_gemm(x, self.packed, self.scales, self.zeros, buf, locks, *cfg, int(self.silu_mul))
+        # decode calls (M <= 16, captured with the workspace finalize made) use the device's, larger ones their stream's
+        buf, locks = w4_hip.workspace(x.device) if x.shape[0] <= 16 else w4_hip.stream_workspace(x.device)
+        call = ext.w4_gemm
+        if cfg[0] == "tiled":
+            call, cfg = ext.w4_gemm_tiled, cfg[1:]
+        return call(x, self.packed, self.scales, self.zeros, buf, locks, *cfg, int(self.silu_mul))
+
+    def gemm_entry(self, m: int, x: torch.Tensor | None = None) -> W4Gemm | None:
+        """The M > 16 kernel: the shape's ladder up to its last m_max, then w4_plan's rule on the sizes (for an x
+        that autograd or a transform follows: None, dequantize + F.linear)."""
+        key = (self.out_features, self.in_features) + (("silu",) if self.silu_mul else ())
+        ladder = self.gemm_kernels.get(key, DEFAULT_GEMM)
+        if ladder and m <= ladder[-1][0]:
+            return pick_gemm(ladder, m)
+        if x is not None and not _plain(x):
+            return None
+        return w4_plan.choose(m, self.out_features, self.in_features, self.silu_mul, self.cus)
 
     def kernel_for(self, m: int) -> str:
         """The kernel forward runs for a 16-byte aligned fp16 x of M rows on the GPU, by the same
@@ -302,11 +322,10 @@ class W4Linear(nn.Module):
             if kind not in ("gemm", "mmak", "mmap", "mma", "gemvm") and not (kind == "gemv" and m <= 4):
                 kind, *cfg = DEFAULT_KERNEL
             return f"{kind}{tuple(cfg)}"
-        key = (self.out_features, self.in_features) + (("silu",) if self.silu_mul else ())
-        cfg = pick_gemm(self.gemm_kernels.get(key, DEFAULT_GEMM), m)
+        cfg = self.gemm_entry(m)
         if not FUSED_GEMM or cfg is None or m * self.in_features >= 1 << 31 or (cfg[0] == "mma" and m > 64):
             return "dequant+matmul"
-        return f"mma{tuple(cfg[1:])}" if cfg[0] == "mma" else f"gemm{tuple(cfg)}"
+        return f"{cfg[0]}{tuple(cfg[1:])}" if cfg[0] in ("mma", "tiled") else f"gemm{tuple(cfg)}"
 
     def decode_entry(self, m: int) -> W4Kernel:
         """The table entry forward uses at 1 <= M <= 16."""
@@ -386,8 +405,7 @@ class W4Linear(nn.Module):
         elif _gemm_ok(x):  # M > 16: the GEMM, unless the table prefers dequantize + torch.matmul
             ext = w4_hip.load()
             if ext is not None:
-                key = (self.out_features, self.in_features) + (("silu",) if self.silu_mul else ())
-                cfg = pick_gemm(self.gemm_kernels.get(key, DEFAULT_GEMM), x.shape[0])
+                cfg = self.gemm_entry(x.shape[0], x)
                 if cfg is not None and cfg[0] == "mma" and x.shape[0] <= 64:  # the streaming kernel, M <= 64
                     return ext.w4_mma(x, self.packed, self.scales, self.zeros, *cfg[1:], int(self.silu_mul))
                 if cfg is not None and cfg[0] != "mma":

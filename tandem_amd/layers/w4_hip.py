@@ -29,6 +29,8 @@ TW4_OK, TW4_EINVAL, TW4_ECONFIG, TW4_EHIP, TW4_ESPACE = 0, 1, 2, 3, 4
 WORKSPACE_FLOATS = 1 << 23  # 32 MB of float32 split-K partial sums per GPU (w4_cuda.py:24)
 WORKSPACE_LOCKS = 1 << 15
 _workspaces: dict[int, tuple[torch.Tensor, torch.Tensor]] = {}
+STREAM_WORKSPACES = 8  # at most this many per-stream workspaces are kept, the oldest given back first
+_stream_workspaces: dict[tuple[int, int, int], tuple[torch.Tensor, torch.Tensor]] = {}
 _init_lock = threading.Lock()
 _initialized: set[int] = set()
 
@@ -50,6 +52,9 @@ _SIGNATURES = {
     "tw4_mma_persist": ([_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _P], _I),
     "tw4_gemm": ([_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P], _I),
     "tw4_gemm_noalloc": ([_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P], _I),
+    "tw4_capture_id": ([_P], ctypes.c_uint64),
+    "tw4_gemm_tiled": ([_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P], _I),
+    "tw4_gemm_tiled_configs": ([ctypes.POINTER(_I), _I], _I),
     "tw4_gemm_last_grid": ([ctypes.POINTER(_I)] * 3, _I),
     "tw4_read_probe": ([_P, _I64, _I, _I, _I, ctypes.c_uint32, _P, _P], _I),
     "tw4_decode_configs": ([ctypes.POINTER(_I), _I], _I),
@@ -106,6 +111,11 @@ def gemm_configs() -> tuple[tuple[int, int, int, int, int], ...]:
 
 
 def gemv_f16_configs() -> tuple[tuple[int, int], ...]:
+def gemm_tiled_configs() -> tuple[tuple[int, int, int, int, int, int], ...]:
+    """The compiled (mt, nt, warps_n, warps_m, warps_k, ring) configurations of w4_gemm_tiled."""
+    return _configs("tw4_gemm_tiled_configs", 6)
+
+
     """The compiled (rows in flight, rows per wavefront) configurations of tw4_gemv_f16."""
     return _configs("tw4_gemv_f16_configs", 2)
 
@@ -290,6 +300,28 @@ class W4Extension:
         return y
 
     def w4_gemm_noalloc(self, x, w, s, z, mt: int, nt: int, warps_n: int, warps_k: int, stages: int, splits: int,
+    def w4_gemm_tiled(self, x, w, s, z, ws, locks, mt: int, nt: int, warps_n: int, warps_m: int, warps_k: int, ring: int,
+                      splits: int, act: int) -> torch.Tensor:
+        """w4_gemm with both tiles through LDS, any compiled tile and ring depth (gemm_tiled_configs), N % 8 == 0."""
+        m, n, k = check_operands("w4_gemm", x, w, s, z)
+        if not (ws.is_cuda and ws.dtype == torch.float32 and locks.is_cuda and locks.dtype == torch.int32
+                and ws.device == x.device and locks.device == x.device and ws.is_contiguous()
+                and locks.is_contiguous()):
+            raise RuntimeError("w4_gemm: float32 workspace and int32 locks (zero) on x's GPU")
+        if act not in (0, 1) or (act and n % 16):
+            raise RuntimeError("w4_gemm: act 0, or 1 (SwiGLU) with N % 16 == 0")
+        if m * k >= 1 << 31:
+            raise RuntimeError("w4_gemm: M x K < 2^31")
+        y = torch.empty((m, n // 2 if act else n), dtype=torch.float16, device=x.device)
+        if m == 0:
+            return y
+        with torch.cuda.device(x.device):
+            init_device(x.device)
+            check(self.lib.tw4_gemm_tiled(_ptr(x), _ptr(w), _ptr(s), _ptr(z), _ptr(y), _ptr(ws), _ptr(locks),
+                                          ws.numel(), locks.numel(), m, n, k, int(mt), int(nt), int(warps_n),
+                                          int(warps_m), int(warps_k), int(ring), int(splits), int(act), _stream(x)))
+        return y
+
                         act: int, out: torch.Tensor | None = None) -> torch.Tensor:
         """w4_gemm with the library's static split-K scratch instead of a workspace (tw4_gemm_noalloc: the
         C entry point allocates nothing). y comes from ``out`` (float16 [M, N] or [M, N / 2], contiguous,
@@ -394,6 +426,28 @@ def workspace(device: torch.device | str | int) -> tuple[torch.Tensor, torch.Ten
 
 
 @functools.lru_cache(maxsize=None)
+def stream_workspace(device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
+    """``workspace`` for the current stream alone, so calls on several streams (or threads with a stream each) and
+    graphs replayed side by side share no partial sums: one per stream, and one per graph capture, which takes it from
+    the graph's own memory and clears its counters there. A buffer given back returns to its stream's (its graph's) pool,
+    where whatever takes it next is ordered behind the kernels that used it."""
+    index = device.index if device.index is not None else torch.cuda.current_device()
+    stream = torch.cuda.current_stream(index).cuda_stream
+    capture = library().tw4_capture_id(stream) if stream else 0
+    key = (index, stream, capture)
+    buf = _stream_workspaces.get(key)
+    if buf is None:
+        with _init_lock:
+            for old in [k for k in _stream_workspaces if capture and k[2]]:  # one capture's at a time
+                del _stream_workspaces[old]
+            while len(_stream_workspaces) >= STREAM_WORKSPACES:
+                del _stream_workspaces[next(iter(_stream_workspaces))]
+            dev = torch.device("cuda", index)
+            buf = _stream_workspaces[key] = (torch.empty(WORKSPACE_FLOATS, dtype=torch.float32, device=dev),
+                                             torch.zeros(WORKSPACE_LOCKS, dtype=torch.int32, device=dev))
+    return buf
+
+
 def load() -> W4Extension | None:
     """The fused W4A16 kernels, or None when TANDEM_NO_CUDA_EXT=1 switches them off (the layer then
     dequantizes with the HIP kernel and multiplies with torch.matmul). Raises if the library is
