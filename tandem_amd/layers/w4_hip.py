@@ -110,12 +110,12 @@ def gemm_configs() -> tuple[tuple[int, int, int, int, int], ...]:
     return _configs("tw4_gemm_configs", 5)
 
 
-def gemv_f16_configs() -> tuple[tuple[int, int], ...]:
 def gemm_tiled_configs() -> tuple[tuple[int, int, int, int, int, int], ...]:
     """The compiled (mt, nt, warps_n, warps_m, warps_k, ring) configurations of w4_gemm_tiled."""
     return _configs("tw4_gemm_tiled_configs", 6)
 
 
+def gemv_f16_configs() -> tuple[tuple[int, int], ...]:
     """The compiled (rows in flight, rows per wavefront) configurations of tw4_gemv_f16."""
     return _configs("tw4_gemv_f16_configs", 2)
 
@@ -299,7 +299,6 @@ class W4Extension:
                                     int(warps_k), int(stages), int(splits), int(act), _stream(x)))
         return y
 
-    def w4_gemm_noalloc(self, x, w, s, z, mt: int, nt: int, warps_n: int, warps_k: int, stages: int, splits: int,
     def w4_gemm_tiled(self, x, w, s, z, ws, locks, mt: int, nt: int, warps_n: int, warps_m: int, warps_k: int, ring: int,
                       splits: int, act: int) -> torch.Tensor:
         """w4_gemm with both tiles through LDS, any compiled tile and ring depth (gemm_tiled_configs), N % 8 == 0."""
@@ -322,6 +321,7 @@ class W4Extension:
                                           int(warps_m), int(warps_k), int(ring), int(splits), int(act), _stream(x)))
         return y
 
+    def w4_gemm_noalloc(self, x, w, s, z, mt: int, nt: int, warps_n: int, warps_k: int, stages: int, splits: int,
                         act: int, out: torch.Tensor | None = None) -> torch.Tensor:
         """w4_gemm with the library's static split-K scratch instead of a workspace (tw4_gemm_noalloc: the
         C entry point allocates nothing). y comes from ``out`` (float16 [M, N] or [M, N / 2], contiguous,
@@ -425,7 +425,6 @@ def workspace(device: torch.device | str | int) -> tuple[torch.Tensor, torch.Ten
     return buf
 
 
-@functools.lru_cache(maxsize=None)
 def stream_workspace(device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
     """``workspace`` for the current stream alone, so calls on several streams (or threads with a stream each) and
     graphs replayed side by side share no partial sums: one per stream, and one per graph capture, which takes it from
@@ -448,6 +447,7 @@ def stream_workspace(device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
     return buf
 
 
+@functools.lru_cache(maxsize=None)
 def load() -> W4Extension | None:
     """The fused W4A16 kernels, or None when TANDEM_NO_CUDA_EXT=1 switches them off (the layer then
     dequantizes with the HIP kernel and multiplies with torch.matmul). Raises if the library is
