@@ -209,8 +209,8 @@ int tw4_gemm(const uint16_t* x, const int32_t* packed, const uint16_t* scales,
  * N % 8 == 0 with scales and zeros 4-byte aligned. BM = 16 mt warps_m tokens, BN = 16 nt warps_n rows, `ring` stages
  * of 64 k in LDS, warps_k 1, or 2: two wavefronts per (tokens, rows) part, each with half of every stage. splits: 0 as
  * for stages 3, 1, or that many contiguous ranges of whole quant groups per tile (at most 2 K / 128; a range past the
- * groups is empty). Otherwise tw4_gemm's contract. No reference counterpart
- * beyond w4_gemm's (python/tandem/csrc/w4_gemv.cu:312-566). */
+ * groups is empty). Otherwise tw4_gemm's contract. No reference counterpart beyond
+ * w4_gemm's (python/tandem/csrc/w4_gemv.cu:312-566). */
 int tw4_gemm_tiled(const uint16_t* x, const int32_t* packed, const uint16_t* scales,
                    const uint16_t* zeros, uint16_t* y, float* ws, int32_t* locks,
                    int64_t ws_floats, int64_t n_locks, int M, int N, int K,
@@ -249,6 +249,12 @@ int tw4_gemm_noalloc(const uint16_t* x, const int32_t* packed, const uint16_t* s
  * Replaces gemv / _gemv_kernel (python/tandem/layers/triton_gemv.py:26-61, 180-218). */
 int tw4_gemv_f16(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int N, int K,
                  int rows_inflight, int rows_per_wave, void* stream);
+
+/* Dense fp16 product for small batches, bound by streaming w once: y [M, N] = x [M, K] @ w [N, K]^T, 1 <= M <= 32,
+ * K % 64 == 0, N K < 2^31, fp32 accumulation; x and w 16-byte aligned. Both operands go through LDS by
+ * direct-to-LDS loads. For the fp16 lm_head at the batches and widths tw4_gemv_f16 does not take.
+ * No reference counterpart (triton_gemv.py stops at M = 8 and leaves the rest to cuBLAS, :285-297). */
+int tw4_gemm_f16(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int N, int K, void* stream);
 
 /* Compiled (rows_inflight, rows_per_wave) configurations of tw4_gemv_f16; returns how many. */
 int tw4_gemv_f16_configs(int* out, int max_configs);

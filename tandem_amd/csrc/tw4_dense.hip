@@ -14,7 +14,7 @@
 // it LDS-bound; the matrix-core form (rows_inflight = 16 or 32: one or two 128-k chunks per step in
 // flight) takes 16-row tiles of w as the A operand of v_mfma_f32_16x16x32_f16 and x as B, so one
 // 16-byte B fragment serves 16 rows.
-#include "tw4_common.h"
+#include "tw4_lds.h"
 
 namespace tw4 {
 
@@ -222,6 +222,124 @@ __global__ void __launch_bounds__(kMmaWaves * 64) dense_mma_kernel(const h1* __r
     }
 }
 
+// ------------------------------------------------------------------- matrix cores through LDS, M <= 32
+// y = x w^T for a batch of up to 32 tokens, bound by streaming w once. Both operands go through LDS by direct-to-LDS
+// loads in a ring of R stages of 64 k, so the loads of w are whole 128-byte lines (the form above reads 64 bytes of
+// 16 rows 2 K bytes apart per instruction), no register holds data in flight, and x is read from LDS by the four
+// wavefronts, 16 rows of w each.
+//   A persistent workgroup owns a contiguous, even share of the 16-row tiles (a grid of one workgroup per 64 rows leaves
+//   its last round nearly empty), and walks it in passes of 64 rows; the stages of all passes form one sequence, so the
+//   loads of the next pass are in flight under the end of this one. Rows past the share repeat its last one (cached; never
+//   stored).
+//   A stage: 64 rows of w and 16 MT of x, 128 bytes per row, 8 rows per load instruction; 16-byte chunk c of row rho at
+//   position c ^ ((rho >> 1) & 7), so the 16 rows of a fragment read touch every bank once.
+//   Lane (q, r) feeds A row r and B column r chunk 4 j + q at substep j. D lane (q, r): rows 4 q + i of token r.
+// What is left to the floor is x: 64 rows of w take 16 MT K 2 bytes of it from L2. Measured on the Qwen3-8B head
+// (4096 x 151936, floor at 7.1 TB/s 175 us), hipBLASLt in the same run in brackets: M = 8 197 us (248; the form above 231),
+// 24 212 (260), 32 221 (265). Timed and not kept: passes of 128 rows (two tiles per wavefront: half of x's traffic, but a
+// ring of 4; M = 8 218 against 204, M = 24 226 against 214 in one run), a ring of 4 stages (209, 218), and 48 and 64 tokens
+// (254 and 273: level with hipBLASLt).
+template <int MT, int R>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
+dense_skinny_kernel(const h1* __restrict__ x, const h1* __restrict__ w, h1* __restrict__ y, int M, int N, int K) {
+    constexpr int ROWS = 64;                  // rows of w per pass
+    constexpr int XL = 2 * MT;                // 1 KB loads of x per stage, 8 rows each
+    constexpr int XI = (XL + 3) / 4, WI = 2;  // per wavefront (the last ones may repeat a load of x)
+    constexpr int SLOT = (ROWS + 16 * MT) * 8;
+    __shared__ u4 ring[R * SLOT];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int tiles = (N + 15) >> 4;
+    const int t0 = static_cast<int>(static_cast<int64_t>(blockIdx.x) * tiles / gridDim.x);
+    const int t1 = static_cast<int>(static_cast<int64_t>(blockIdx.x + 1) * tiles / gridDim.x);
+    const int row_end = min(16 * t1, N), passes = (t1 - t0 + 3) >> 2, ks = K >> 6;
+    if (passes == 0) return;
+
+    const u4 xr = lds_rsrc(x);
+    u4 wr = lds_rsrc(w);
+    const int rho = lane >> 3;  // row of this lane within a load
+    uint32_t xoff[XI], woff[WI];
+    const int xj = min(wave * XI, XL - XI);
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int row = 8 * (xj + i) + rho;
+        xoff[i] = static_cast<uint32_t>(min(row, M - 1)) * K * 2u + 16u * ((lane & 7) ^ ((row >> 1) & 7));
+    }
+    auto pass_rows = [&](int p) {
+#pragma unroll
+        for (int i = 0; i < WI; ++i) {
+            const int row = 8 * (wave * WI + i) + rho;
+            woff[i] = static_cast<uint32_t>(min(16 * t0 + ROWS * p + row, row_end - 1)) * static_cast<uint32_t>(K) * 2u +
+                      16u * ((lane & 7) ^ ((row >> 1) & 7));
+        }
+    };
+    pass_rows(0);
+    const uint32_t ring_addr = static_cast<uint32_t>(reinterpret_cast<size_t>((lds_void*)ring));
+    const uint32_t wbase = ring_addr + 1024 * wave * WI, xbase = ring_addr + 16 * 8 * ROWS + 1024 * xj;
+
+    int ip = 0, is = 0, islot = 0;  // the next stage to issue: pass, stage of the pass, ring slot
+    auto issue = [&]() {
+        const uint32_t s = 16 * SLOT * islot, soff = 128 * is;
+        lds_dma16<0, true>(wr, woff[0], soff, wbase + s);
+        lds_dma16<1024, true>(wr, woff[1], soff, wbase + s);
+        lds_dma16<0>(xr, xoff[0], soff, xbase + s);
+        islot = islot + 1 == R ? 0 : islot + 1;
+        if (++is == ks) {
+            is = 0, ++ip;
+            if (ip < passes)
+                pass_rows(ip);
+            else
+                wr.z = 0;  // past the end: empty loads keep the counts
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < R - 1; ++i) issue();
+
+    // fragment addresses in a slot (16-byte units): substep j at ^ 4 (chunk 4 j + q)
+    const int sw = (r >> 1) & 7;
+    const int wl = (16 * wave + r) * 8, xl = ROWS * 8 + r * 8;
+    const int c0 = q ^ sw, c1 = (q + 4) ^ sw;
+    int slot = 0;
+    for (int p = 0; p < passes; ++p) {
+        f4 acc[MT];
+#pragma unroll
+        for (int b = 0; b < MT; ++b) acc[b] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        for (int s = 0; s < ks; ++s) {
+            wait_stage<(R - 2) * (XI + WI)>();  // this stage has landed (the stores of a pass's end only make it stricter)
+            ring_barrier();                     // in every wavefront, and nobody reads the slot of the stage before any more
+            issue();
+            const u4* sl = ring + slot * SLOT;
+            slot = slot + 1 == R ? 0 : slot + 1;
+            const h8 a0 = bitcast<h8>(sl[wl + c0]), a1 = bitcast<h8>(sl[wl + c1]);
+            h8 b0[MT], b1[MT];
+#pragma unroll
+            for (int b = 0; b < MT; ++b) b0[b] = bitcast<h8>(sl[xl + 128 * b + c0]), b1[b] = bitcast<h8>(sl[xl + 128 * b + c1]);
+#pragma unroll
+            for (int b = 0; b < MT; ++b) acc[b] = mfma16x16x32(a0, b0[b], acc[b]);
+#pragma unroll
+            for (int b = 0; b < MT; ++b) acc[b] = mfma16x16x32(a1, b1[b], acc[b]);
+        }
+        const bool wide = (N & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 7) == 0;
+        const int n = 16 * t0 + ROWS * p + 16 * wave + 4 * q;
+#pragma unroll
+        for (int b = 0; b < MT; ++b) {
+            const int m = 16 * b + r;
+            if (m >= M || n >= row_end) continue;
+            h1* yp = y + static_cast<int64_t>(m) * N + n;
+            const f4 v = acc[b];
+            if (wide) {  // n + 3 < row_end: both are multiples of 4
+                *reinterpret_cast<h4*>(yp) = h4{static_cast<h1>(v.x), static_cast<h1>(v.y), static_cast<h1>(v.z), static_cast<h1>(v.w)};
+            } else {
+                const float e[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (n + i < row_end) yp[i] = static_cast<h1>(e[i]);
+            }
+        }
+    }
+    wait_stage<0>();  // the empty loads past the end still write their slots
+}
+
 // Compiled (rows in flight RB, rows per wavefront) configurations.
 #define TW4_DENSE_CONFIGS(X) X(1, 16) X(1, 32) X(2, 16) X(2, 32) X(2, 64) X(4, 32) X(4, 64)
 // Matrix-core form (rows_inflight 16 D: 16-row tiles, D chunks of 128 k per step in flight): rows
@@ -279,6 +397,19 @@ int dense_mma(const h1* x, const u4* w, h1* y, int M, int N, int K, int rows_per
     return TW4_EINVAL;
 }
 
+template <int MT, int R>
+int skinny_launch(const h1* x, const h1* w, h1* y, int M, int N, int K, hipStream_t st) {
+    int dev = 0, cus = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess) return tw4host::hip_fail(e, "gemm_f16: device");
+    const int tiles = (N + 15) >> 4;
+    const int grid = tiles < 2 * cus ? tiles : 2 * cus;  // two workgroups fit a CU's LDS
+    dense_skinny_kernel<MT, R><<<static_cast<unsigned>(grid), 256, 0, st>>>(x, w, y, M, N, K);
+    TW4_LAUNCH_CHECK("gemm_f16: launch");
+    return TW4_OK;
+}
+
 template <int RB>
 int dense_by_m(const h1* x, const u4* w, h1* y, int M, int N, int K, int rows_per_wave, hipStream_t st) {
     if (M == 1) return dense_by_k<1, RB>(x, w, y, M, N, K, rows_per_wave, st);
@@ -330,4 +461,21 @@ extern "C" int tw4_gemv_f16_configs(int* out, int max_configs) {
     TW4_DENSE_MMA_CONFIGS(TW4_LIST)
 #undef TW4_LIST
     return n;
+}
+
+extern "C" int tw4_gemm_f16(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int N, int K, void* stream) {
+    TW4_REQUIRE(x && w && y, TW4_EINVAL, "gemm_f16: null pointer");
+    TW4_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(w) % 16 == 0, TW4_EINVAL,
+                "gemm_f16: x and w must be 16-byte aligned");
+    TW4_REQUIRE(reinterpret_cast<uintptr_t>(y) % 2 == 0, TW4_EINVAL, "gemm_f16: y must be 2-byte aligned");
+    TW4_REQUIRE(M >= 1 && M <= 32, TW4_EINVAL, "gemm_f16: 1 <= M <= 32 (M = %d)", M);
+    TW4_REQUIRE(N >= 1, TW4_EINVAL, "gemm_f16: N >= 1 (N = %d)", N);
+    TW4_REQUIRE(K >= 64 && K % 64 == 0, TW4_EINVAL, "gemm_f16: K %% 64 == 0 (K = %d)", K);
+    TW4_REQUIRE(static_cast<int64_t>(N) * K < (1LL << 31) && static_cast<int64_t>(M) * K < (1LL << 31), TW4_EINVAL,
+                "gemm_f16: N K < 2^31 (N %d, K %d)", N, K);  // the loads' byte offsets are 32-bit
+    auto xp = reinterpret_cast<const h1*>(x);
+    auto wp = reinterpret_cast<const h1*>(w);
+    auto yp = reinterpret_cast<h1*>(y);
+    auto st = static_cast<hipStream_t>(stream);
+    return M <= 16 ? skinny_launch<1, 7>(xp, wp, yp, M, N, K, st) : skinny_launch<2, 6>(xp, wp, yp, M, N, K, st);
 }

@@ -31,19 +31,15 @@ from tandem_amd.layers import w4_hip
 # gfx architecture.
 Config = tuple[int, int]
 GFX950_DENSE: dict[tuple[int, int, int], Config] = {
-    # Qwen3-8B lm_head: 190 / 185 / 188 us at M = 1 / 2 / 4 (82-84 % of 8 TB/s) vs F.linear 243-251 us;
-    # M = 5 .. 8: the matrix-core form with two chunks in flight, 231 us vs F.linear 246-249 us
-    # (one chunk: 234-239 us; the v_dot2 form: 270-283 us)
+    # Qwen3-8B lm_head: 190 / 185 / 188 us at M = 1 / 2 / 4 (82-84 % of 8 TB/s) vs F.linear 243-251 us
+    # (M = 5 .. 8: no entry, tw4_gemm_f16 by its rule, 196-197 us where the matrix-core form (32, 16) took 231)
     (151936, 4096, 1): (4, 32),
     (151936, 4096, 2): (2, 32),
     (151936, 4096, 4): (2, 32),
-    (151936, 4096, 8): (32, 16),
-    # Qwen3-1.7B lm_head: 96-99 us at M = 1 .. 4, 119 us at M = 8 (the matrix-core form) vs
-    # F.linear 203 us
+    # Qwen3-1.7B lm_head: 96-99 us at M = 1 .. 4 vs F.linear 203 us (M = 5 .. 8: tw4_gemm_f16 107, (16, 16) 116-119)
     (151936, 2048, 1): (2, 16),
     (151936, 2048, 2): (2, 16),
     (151936, 2048, 4): (2, 16),
-    (151936, 2048, 8): (16, 16),
 }
 CONFIGS: dict[str, dict[tuple[int, int, int], Config]] = {
     "AMD Instinct MI355X": GFX950_DENSE,
@@ -124,11 +120,63 @@ def entry(x: torch.Tensor, w: torch.Tensor, table: dict[tuple[int, int, int], Co
     return table.get((w.shape[0], w.shape[1], m_bucket(x.shape[0])))
 
 
+def gemm(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """y [M, N] = x [M, K] @ w [N, K]^T by tw4_gemm_f16, 1 <= M <= 32, K a multiple of 64, contiguous 16-byte aligned
+    float16 tensors on one GPU, on the current stream."""
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1]:
+        raise ValueError(f"gemm: x [M, K] and w [N, K] expected (x {tuple(x.shape)}, w {tuple(w.shape)})")
+    for name, t in (("x", x), ("w", w)):
+        if not (t.is_cuda and t.dtype == torch.float16 and t.is_contiguous() and t.data_ptr() % 16 == 0):
+            raise RuntimeError(f"gemm: {name} must be a contiguous 16-byte aligned float16 GPU tensor")
+    if w.device != x.device:
+        raise RuntimeError("gemm: x and w must be on one GPU")
+    (m, k), n = x.shape, w.shape[0]
+    out = torch.empty((m, n), dtype=torch.float16, device=x.device)
+    with torch.cuda.device(x.device):
+        w4_hip.check(w4_hip.library().tw4_gemm_f16(x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k,
+                                                   torch.cuda.current_stream(x.device).cuda_stream))
+    return out
+
+
+# Where tw4_gemm_f16 (and tw4_gemv_f16 up to M = 4) takes a product no table entry names: weights of at least this many
+# bytes and at most 32 rows. Against F.linear (hipBLASLt) on MI355X, us: 1.24 GB (4096 x 151936) 197 / 212 / 221 at M = 8 / 24
+# / 32 against 248 / 260 / 265, 0.78 GB (2560 wide) 120 / 136 / 148 against 244 / 166 / 168, 134 MB (4096 x 16384) 28.6-29.5
+# against 32; at 67 MB (4096 x 8192, 2048 x 16384) launch and first loads decide and hipBLASLt is ahead (22 against 15,
+# 16.3 against 15.0), and at 48 rows x from L2 makes it level (250 against 252).
+GEMM_MIN_BYTES = 128 << 20
+GEMM_MAX_ROWS = 32
+
+
+def _streams(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether F.linear(x, w) is a product bound by streaming w that tw4_gemm_f16 takes: up to
+    GEMM_MAX_ROWS rows, at least GEMM_MIN_BYTES of weights (and N K < 2^31), K a multiple of 64, plain contiguous aligned
+    float16 GPU tensors that no gradient or transform follows."""
+    if x.dim() != 2 or w.dim() != 2 or not 1 <= x.shape[0] <= GEMM_MAX_ROWS:
+        return False
+    if x.dtype != torch.float16 or w.dtype != torch.float16:
+        return False
+    n, k = w.shape
+    if k % 64 or x.shape[1] != k or not GEMM_MIN_BYTES <= 2 * n * k < 1 << 32 or not x.is_cuda or w.device != x.device:
+        return False
+    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
+        return False
+    wrapped = torch._C._functorch.is_functorch_wrapped_tensor
+    if wrapped(x) or wrapped(w) or not x.is_contiguous() or not w.is_contiguous():
+        return False
+    return x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
+
+
 def linear(x: torch.Tensor, w: torch.Tensor, table: dict[tuple[int, int, int], Config],
            eager: bool = True) -> torch.Tensor:
-    """F.linear(x, w) (no bias) through tw4_gemv_f16 where ``entry`` finds a configuration, through
-    F.linear (hipBLASLt) otherwise (python/tandem/layers/triton_gemv.py:285-297)."""
+    """F.linear(x, w) (no bias) through tw4_gemv_f16 where ``entry`` finds a configuration, on a GPU with a table through
+    tw4_gemm_f16 where streaming w bounds it (the logits head at every other batch up to 32 and every other size; up to
+    M = 4, whose x the vector form keeps in LDS whole, tw4_gemv_f16 where it takes K: 184 us against 197 on the Qwen3-8B
+    head at M = 1), through F.linear (hipBLASLt) otherwise (python/tandem/layers/triton_gemv.py:285-297)."""
     cfg = entry(x, w, table, eager)
+    if cfg is None and eager and table and _streams(x, w):
+        if x.shape[0] > 4 or x.shape[1] not in KS:
+            return gemm(x, w)
+        cfg = (2, 32) if w.shape[0] >= 1 << 16 else (2, 16)  # rows per wavefront: enough wavefronts for the GPU
     return F.linear(x, w) if cfg is None else gemv(x, w, *cfg)
 
 
