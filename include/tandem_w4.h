@@ -259,6 +259,12 @@ int tw4_gemm_f16(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int N
 /* Compiled (rows_inflight, rows_per_wave) configurations of tw4_gemv_f16; returns how many. */
 int tw4_gemv_f16_configs(int* out, int max_configs);
 
+/* Attention over a one-token context (softmax over a single key is 1): query head h of a token takes the value row of KV
+ * head h / (heads / kv_heads). qkv fp16 [M, (heads + 2 kv_heads) head_dim] = [q | k | v] -> y fp16 [M, heads head_dim];
+ * head_dim % 8 == 0, heads % kv_heads == 0, both 16-byte aligned. Stands where the reference's attention backend
+ * runs (python/tandem/layers/attention.py). */
+int tw4_attend_one(const uint16_t* qkv, uint16_t* y, int M, int heads, int kv_heads, int head_dim, void* stream);
+
 /* RMSNorm of the decoder layer around the projections, fp16 rows [M, K], fp32 math, K % 512 == 0,
  * K <= 8192, rows 16-byte aligned. y = fp16(x * rsqrt(mean(x^2) + eps) * weight).
  * Replaces ops.rms_norm of the GPU path (python/tandem/layers/ops.py:107-109, FlashInfer's

@@ -222,7 +222,7 @@ def _table(tables: dict, device_name: str | None, device: torch.device) -> dict:
     return {}
 
 
-def _plain(x: torch.Tensor) -> bool:
+def plain(x: torch.Tensor) -> bool:
     """No gradient is asked of x and no transform (vmap, jvp) wraps it: a call that dequantize + F.linear would have to
     carry through autograd or a transform must not go to a kernel that sees a data pointer only."""
     return not (x.requires_grad and torch.is_grad_enabled()) and not torch._C._functorch.is_functorch_wrapped_tensor(x)
@@ -308,7 +308,7 @@ class W4Linear(nn.Module):
         ladder = self.gemm_kernels.get(key, DEFAULT_GEMM)
         if ladder and m <= ladder[-1][0]:
             return pick_gemm(ladder, m)
-        if x is not None and not _plain(x):
+        if x is not None and not plain(x):
             return None
         return w4_plan.choose(m, self.out_features, self.in_features, self.silu_mul, self.cus)
 

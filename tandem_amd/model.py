@@ -32,7 +32,7 @@ from typing import Any, Optional
 import torch
 from torch import nn
 
-from tandem_amd.layers import gemv16, norm
+from tandem_amd.layers import awq, gemv16, norm, w4_hip
 from tandem_amd.layers.linear import finalize_quantized, make_linear
 
 
@@ -101,10 +101,25 @@ class Attention(nn.Module):
         self.qkv_proj = make_linear(cfg.hidden_size, self.q_size + 2 * self.kv_size, False, quant)
         self.o_proj = make_linear(self.q_size, cfg.hidden_size, False, quant)
 
+    def _hip_attend(self, qkv: torch.Tensor) -> bool:
+        """Plain contiguous 16-byte aligned fp16 GPU rows [q | k | v] that no gradient or transform follows, whole 16-byte
+        chunks per head: tw4_attend_one; anything else the torch expression of the same copy."""
+        return (qkv.is_cuda and qkv.dtype == torch.float16 and qkv.dim() == 2 and qkv.numel() > 0 and qkv.is_contiguous()
+                and qkv.shape[1] == self.q_size + 2 * self.kv_size and self.head_dim % 8 == 0
+                and self.num_heads % self.num_kv_heads == 0 and qkv.data_ptr() % 16 == 0
+                and 8 * (1 << 31) > qkv.numel() and awq.plain(qkv))
+
     def attend(self, qkv: torch.Tensor) -> torch.Tensor:
         """[M, q | k | v] -> [M, num_heads * head_dim]: query head h takes the value row of KV head
         h // (num_heads / num_kv_heads)."""
         m = qkv.shape[0]
+        if self._hip_attend(qkv):
+            y = torch.empty((m, self.q_size), dtype=torch.float16, device=qkv.device)
+            with torch.cuda.device(qkv.device):
+                w4_hip.check(w4_hip.library().tw4_attend_one(
+                    qkv.data_ptr(), y.data_ptr(), m, self.num_heads, self.num_kv_heads, self.head_dim,
+                    torch.cuda.current_stream(qkv.device).cuda_stream))
+            return y
         v = qkv[:, self.q_size + self.kv_size:].view(m, self.num_kv_heads, 1, self.head_dim)
         group = self.num_heads // self.num_kv_heads
         return v.expand(m, self.num_kv_heads, group, self.head_dim).reshape(m, self.q_size).contiguous()
