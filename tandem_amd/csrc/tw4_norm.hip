@@ -4,82 +4,82 @@
 //   tw4_rms_norm:      y = fp16(x rstd w),                  rstd = rsqrt(mean(x^2) + eps)
 //   tw4_add_rms_norm:  s = x + r (fp32); r <- fp16(s); x <- fp16(s rstd w),  rstd from s (in place)
 //
-// One wavefront per row: lane l holds chunks (8 halves, 16 bytes) l, l + 64, ... of the row, all
-// loaded before any math (J = K / 512 chunks per lane, kept in registers for the second pass). The
-// sum of squares follows the fixed order of norm_rstd (per chunk, per quant group of 16 chunks, then
-// over the groups), the same order as the decode kernels' fused norm prologue, so a fused
-// projection sees the very bits this kernel writes. A decode batch is a few rows: the kernel is
-// latency-bound (two dependent memory round trips), 4 rows per workgroup.
+// A workgroup per row, W wavefronts of J chunks per lane (8 halves, 16 bytes: chunks W 64 j + 64 wave + lane of the row),
+// all loaded before any math and kept in registers for the second pass. The sum of squares follows the fixed order of
+// norm_rstd (per chunk, per quant group of 16 chunks, then over the groups), the same order as the decode kernels' fused
+// norm prologue, so a fused projection sees the very bits this kernel writes.
+// A decode batch is a few rows and latency-bound: one chunk per lane (two from K = 5120) leaves two dependent round trips to
+// memory and one chunk's arithmetic, where a wavefront per row ran all K / 512 chunks' one after another. us before ->
+// after, add + norm (norm alone): K 4096 M = 1 2.7 -> 1.9 (2.5 -> 1.8), M = 8 3.4 -> 2.1 (3.0 -> 2.0), M = 512 4.4 -> 3.5;
+// K 2048 M = 5 2.3 -> 1.9; K 5120 M = 40 3.9 -> 2.3; K 8192 M = 8 5.3 -> 2.4. The launch itself takes 1.8.
+// From kTallRows rows on the rows alone fill the GPU and the kernel is bound by memory: fewer wavefronts per row with more
+// loads in flight each. add + norm at M = 2048, that form / the short one / a wavefront per row: K 2560 5.5 / 5.7 / 5.6,
+// K 4096 7.5 / 7.6 / 8.1, K 5120 10.9 / 11.6 / 10.8.
 #include "tw4_common.h"
 
 namespace tw4 {
 
 constexpr int kNormMaxGroups = 64;  // K <= 8192
+constexpr int kTallRows = 1024;
 
-template <bool ADD, int J>
-__global__ void __launch_bounds__(256) rms_norm_kernel(h1* x, h1* r, const h1* __restrict__ w, h1* y, int M, int K,
-                                                       float eps) {  // y may be x: every store follows every load
-    __shared__ float gsum[4][kNormMaxGroups];
+template <bool ADD, int W, int J>
+__global__ void __launch_bounds__(64 * W) rms_norm_kernel(h1* x, h1* r, const h1* __restrict__ w, h1* y, int K,
+                                                          float eps) {  // y may be x: every store follows every load
+    __shared__ float gsum[kNormMaxGroups];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int row = blockIdx.x * 4 + wave;
-    if (row >= M) return;  // whole wavefronts; no workgroup barrier below
-    const int64_t base = static_cast<int64_t>(row) * (K >> 3);
+    const int64_t base = static_cast<int64_t>(blockIdx.x) * (K >> 3);
     u4* xr = reinterpret_cast<u4*>(x) + base;
     u4* rr = reinterpret_cast<u4*>(r) + base;
     const u4* wr = reinterpret_cast<const u4*>(w);
     u4 xv[J], rv[J], wv[J];
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-        xv[j] = xr[64 * j + lane];
-        if constexpr (ADD) rv[j] = rr[64 * j + lane];
-        wv[j] = wr[64 * j + lane];
+        const int c = 64 * W * j + threadIdx.x;
+        xv[j] = xr[c];
+        if constexpr (ADD) rv[j] = rr[c];
+        wv[j] = wr[c];
     }
-    float* gs = gsum[wave];
+    float s[J][8];
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-        float s[8];
-        chunk_to_f32(xv[j], s);
+        chunk_to_f32(xv[j], s[j]);
         if constexpr (ADD) {
             float b[8];
             chunk_to_f32(rv[j], b);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) s[i] += b[i];
+            for (int i = 0; i < 8; ++i) s[j][i] += b[i];
         }
-        const float q = row16_sum(sumsq8(s));  // group 4 j + lane / 16
-        if ((lane & 15) == 0) gs[4 * j + (lane >> 4)] = q;
+        const float q = row16_sum(sumsq8(s[j]));  // quant group 4 (W j + wave) + lane / 16
+        if ((lane & 15) == 0) gsum[4 * (W * j + wave) + (lane >> 4)] = q;
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const float rstd = norm_rstd(gs, K >> 7, K, eps, lane);
+    __syncthreads();
+    const float rstd = norm_rstd(gsum, K >> 7, K, eps, lane);
     u4* yr = reinterpret_cast<u4*>(y) + base;
 #pragma unroll
     for (int j = 0; j < J; ++j) {
-        float s[8], g[8];
-        chunk_to_f32(xv[j], s);
-        if constexpr (ADD) {
-            float b[8];
-            chunk_to_f32(rv[j], b);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) s[i] += b[i];
-            rr[64 * j + lane] = f32_to_chunk(s);
-        }
+        const int c = 64 * W * j + threadIdx.x;
+        float g[8];
+        if constexpr (ADD) rr[c] = f32_to_chunk(s[j]);
         chunk_to_f32(wv[j], g);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) s[i] = s[i] * rstd * g[i];
-        yr[64 * j + lane] = f32_to_chunk(s);
+        for (int i = 0; i < 8; ++i) s[j][i] = s[j][i] * rstd * g[i];
+        yr[c] = f32_to_chunk(s[j]);
     }
 }
 
 template <bool ADD>
 int norm_launch(h1* x, h1* r, const h1* w, h1* y, int M, int K, float eps, hipStream_t st) {
-    const unsigned grid = static_cast<unsigned>((M + 3) / 4);
-    switch (K >> 9) {
-#define TW4_NORM_CASE(J) \
-    case J: rms_norm_kernel<ADD, J><<<grid, 256, 0, st>>>(x, r, w, y, M, K, eps); break;
-        TW4_NORM_CASE(1) TW4_NORM_CASE(2) TW4_NORM_CASE(3) TW4_NORM_CASE(4) TW4_NORM_CASE(5)
-        TW4_NORM_CASE(6) TW4_NORM_CASE(7) TW4_NORM_CASE(8) TW4_NORM_CASE(10) TW4_NORM_CASE(12)
-        TW4_NORM_CASE(14) TW4_NORM_CASE(16)
+    const unsigned grid = static_cast<unsigned>(M);
+    const int tall = M >= kTallRows ? 100 : 0;
+    switch (tall + (K >> 9)) {
+#define TW4_NORM_CASE(TALL, W, J) \
+    case TALL + W * J: rms_norm_kernel<ADD, W, J><<<grid, 64 * W, 0, st>>>(x, r, w, y, K, eps); break;
+        TW4_NORM_CASE(0, 1, 1) TW4_NORM_CASE(0, 2, 1) TW4_NORM_CASE(0, 3, 1) TW4_NORM_CASE(0, 4, 1)
+        TW4_NORM_CASE(0, 5, 1) TW4_NORM_CASE(0, 6, 1) TW4_NORM_CASE(0, 7, 1) TW4_NORM_CASE(0, 8, 1)
+        TW4_NORM_CASE(0, 5, 2) TW4_NORM_CASE(0, 6, 2) TW4_NORM_CASE(0, 7, 2) TW4_NORM_CASE(0, 8, 2)
+        TW4_NORM_CASE(100, 1, 1) TW4_NORM_CASE(100, 1, 2) TW4_NORM_CASE(100, 1, 3) TW4_NORM_CASE(100, 2, 2)
+        TW4_NORM_CASE(100, 1, 5) TW4_NORM_CASE(100, 3, 2) TW4_NORM_CASE(100, 1, 7) TW4_NORM_CASE(100, 4, 2)
+        TW4_NORM_CASE(100, 2, 5) TW4_NORM_CASE(100, 4, 3) TW4_NORM_CASE(100, 7, 2) TW4_NORM_CASE(100, 4, 4)
 #undef TW4_NORM_CASE
         default:
             tw4host::set_error("rms_norm: K = %d is not compiled (K / 512 in 1..8, 10, 12, 14, 16)", K);
