@@ -222,12 +222,6 @@ def _table(tables: dict, device_name: str | None, device: torch.device) -> dict:
     return {}
 
 
-def plain(x: torch.Tensor) -> bool:
-    """No gradient is asked of x and no transform (vmap, jvp) wraps it: a call that dequantize + F.linear would have to
-    carry through autograd or a transform must not go to a kernel that sees a data pointer only."""
-    return not (x.requires_grad and torch.is_grad_enabled()) and not torch._C._functorch.is_functorch_wrapped_tensor(x)
-
-
 # Chunks (16 bytes of x) one wavefront stages in one batch: 64 lanes x 2 (kXB in tw4_decode.hip).
 FUSED_NORM_CHUNKS = 128
 
@@ -308,7 +302,7 @@ class W4Linear(nn.Module):
         ladder = self.gemm_kernels.get(key, DEFAULT_GEMM)
         if ladder and m <= ladder[-1][0]:
             return pick_gemm(ladder, m)
-        if x is not None and not plain(x):
+        if x is not None and not w4_hip.plain(x):
             return None
         return w4_plan.choose(m, self.out_features, self.in_features, self.silu_mul, self.cus)
 

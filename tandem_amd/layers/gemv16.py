@@ -158,10 +158,7 @@ def _streams(x: torch.Tensor, w: torch.Tensor) -> bool:
     n, k = w.shape
     if k % 64 or x.shape[1] != k or not GEMM_MIN_BYTES <= 2 * n * k < 1 << 32 or not x.is_cuda or w.device != x.device:
         return False
-    if torch.is_grad_enabled() and (x.requires_grad or w.requires_grad):
-        return False
-    wrapped = torch._C._functorch.is_functorch_wrapped_tensor
-    if wrapped(x) or wrapped(w) or not x.is_contiguous() or not w.is_contiguous():
+    if not (w4_hip.plain(x) and w4_hip.plain(w) and x.is_contiguous() and w.is_contiguous()):
         return False
     return x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0
 

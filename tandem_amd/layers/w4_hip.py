@@ -21,6 +21,7 @@ import os
 import threading
 
 import torch
+from torch.autograd import forward_ad
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lib", "libtandem_w4.so")
 
@@ -447,6 +448,16 @@ def stream_workspace(device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
             buf = _stream_workspaces[key] = (torch.empty(WORKSPACE_FLOATS, dtype=torch.float32, device=dev),
                                              torch.zeros(WORKSPACE_LOCKS, dtype=torch.int32, device=dev))
     return buf
+
+
+def plain(x: torch.Tensor) -> bool:
+    """An ordinary tensor that only the values of this call matter to: no gradient or tangent is asked of it, no transform
+    (vmap, jvp), tracer, compiler or dispatch mode follows the call. Anything else has to stay in torch operators, as a kernel that
+    sees a data pointer only would drop what follows it."""
+    return (type(x) in (torch.Tensor, torch.nn.Parameter) and not (x.requires_grad and torch.is_grad_enabled())
+            and not torch.compiler.is_compiling() and not torch.jit.is_tracing()
+            and not torch._C._len_torch_dispatch_stack() and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+            and forward_ad.unpack_dual(x).tangent is None)
 
 
 @functools.lru_cache(maxsize=None)

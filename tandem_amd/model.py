@@ -32,7 +32,7 @@ from typing import Any, Optional
 import torch
 from torch import nn
 
-from tandem_amd.layers import awq, gemv16, norm, w4_hip
+from tandem_amd.layers import gemv16, norm, w4_hip
 from tandem_amd.layers.linear import finalize_quantized, make_linear
 
 
@@ -104,10 +104,11 @@ class Attention(nn.Module):
     def _hip_attend(self, qkv: torch.Tensor) -> bool:
         """Plain contiguous 16-byte aligned fp16 GPU rows [q | k | v] that no gradient or transform follows, whole 16-byte
         chunks per head: tw4_attend_one; anything else the torch expression of the same copy."""
-        return (qkv.is_cuda and qkv.dtype == torch.float16 and qkv.dim() == 2 and qkv.numel() > 0 and qkv.is_contiguous()
+        return (w4_hip.plain(qkv) and qkv.is_cuda and qkv.dtype == torch.float16 and qkv.dim() == 2 and qkv.numel() > 0
+                and qkv.is_contiguous()
                 and qkv.shape[1] == self.q_size + 2 * self.kv_size and self.head_dim % 8 == 0
                 and self.num_heads % self.num_kv_heads == 0 and qkv.data_ptr() % 16 == 0
-                and 8 * (1 << 31) > qkv.numel() and awq.plain(qkv))
+                and 8 * (1 << 31) > qkv.numel())
 
     def attend(self, qkv: torch.Tensor) -> torch.Tensor:
         """[M, q | k | v] -> [M, num_heads * head_dim]: query head h takes the value row of KV head

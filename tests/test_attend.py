@@ -38,3 +38,30 @@ def test_attend_matches_torch(m, heads, kv, dim):
     x = qkv.cuda().requires_grad_()
     attn.attend(x).float().sum().backward()
     assert float(x.grad.double().sum()) == m * heads * dim
+
+
+def test_plain_is_false_where_torch_follows_the_call():
+    """A kernel behind a data pointer is invisible to gradients, tangents, transforms, tracers and dispatch modes."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.fx.experimental.proxy_tensor import make_fx
+
+    x, seen = torch.randn(2, 8), []
+
+    def look(t):
+        seen.append(w4_hip.plain(t))
+        return t * 2
+
+    assert w4_hip.plain(x) and w4_hip.plain(torch.nn.Parameter(x, requires_grad=False))
+    look(x.clone().requires_grad_())
+    torch.func.vmap(look)(x)
+    torch.func.jvp(look, (x,), (x,))
+    with torch.autograd.forward_ad.dual_level():
+        look(torch.autograd.forward_ad.make_dual(x, x))
+        assert w4_hip.plain(x)
+    torch.jit.trace(look, x, check_trace=False)
+    make_fx(look)(x)
+    with FakeTensorMode() as mode:
+        look(mode.from_tensor(x))
+    assert len(seen) >= 6 and not any(seen), seen
+    with torch.no_grad():
+        assert w4_hip.plain(x.clone().requires_grad_())
