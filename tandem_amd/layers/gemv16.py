@@ -102,7 +102,7 @@ def gemv(x: torch.Tensor, w: torch.Tensor, rows_inflight: int = 2, rows_per_wave
           or not out.is_contiguous() or out.data_ptr() % 16):
         raise RuntimeError(f"gemv: out must be a contiguous 16-byte aligned float16 [{m}, {n}] tensor on x's GPU")
     w4_hip.check(w4_hip.library().tw4_gemv_f16(x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, rows_inflight,
-                                               rows_per_wave, torch.cuda.current_stream(x.device).cuda_stream))
+                                               rows_per_wave, w4_hip.raw_stream(x.get_device())))
     return out
 
 
@@ -132,9 +132,9 @@ def gemm(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         raise RuntimeError("gemm: x and w must be on one GPU")
     (m, k), n = x.shape, w.shape[0]
     out = torch.empty((m, n), dtype=torch.float16, device=x.device)
-    with torch.cuda.device(x.device):
+    with w4_hip.on_device(x.get_device()):
         w4_hip.check(w4_hip.library().tw4_gemm_f16(x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k,
-                                                   torch.cuda.current_stream(x.device).cuda_stream))
+                                                   w4_hip.raw_stream(x.get_device())))
     return out
 
 

@@ -46,9 +46,9 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, out: torch.Tenso
         y = out.view(m, k)
     if m == 0:
         return y.view(shape)
-    with torch.cuda.device(x.device):
+    with w4_hip.on_device(x.get_device()):
         w4_hip.check(w4_hip.library().tw4_rms_norm(x2.data_ptr(), weight.data_ptr(), y.data_ptr(), m, k, float(eps),
-                                                   torch.cuda.current_stream(x.device).cuda_stream))
+                                                   w4_hip.raw_stream(x.get_device())))
     return y.view(shape)
 
 
@@ -62,9 +62,9 @@ def fused_add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Te
         raise RuntimeError("fused_add_rms_norm: residual must match x")
     if m == 0:
         return x, residual
-    with torch.cuda.device(x.device):
+    with w4_hip.on_device(x.get_device()):
         w4_hip.check(w4_hip.library().tw4_add_rms_norm(x.data_ptr(), residual.data_ptr(), weight.data_ptr(), m, k,
-                                                       float(eps), torch.cuda.current_stream(x.device).cuda_stream))
+                                                       float(eps), w4_hip.raw_stream(x.get_device())))
     return x, residual
 
 

@@ -116,10 +116,10 @@ class Attention(nn.Module):
         m = qkv.shape[0]
         if self._hip_attend(qkv):
             y = torch.empty((m, self.q_size), dtype=torch.float16, device=qkv.device)
-            with torch.cuda.device(qkv.device):
+            with w4_hip.on_device(qkv.get_device()):
                 w4_hip.check(w4_hip.library().tw4_attend_one(
                     qkv.data_ptr(), y.data_ptr(), m, self.num_heads, self.num_kv_heads, self.head_dim,
-                    torch.cuda.current_stream(qkv.device).cuda_stream))
+                    w4_hip.raw_stream(qkv.get_device())))
             return y
         v = qkv[:, self.q_size + self.kv_size:].view(m, self.num_kv_heads, 1, self.head_dim)
         group = self.num_heads // self.num_kv_heads
