@@ -152,7 +152,8 @@ def w4_dequant(packed: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor, 
 #                                      staging x once and streaming several row-tile groups, M <= 16
 #   ("gemm", MT, NT, WARPS_N, WARPS_K, STAGES, SPLITS)   the fused GEMM (below), where it wins
 # warps_k: wavefronts splitting K in a workgroup; unroll: quant groups in flight per lane and
-# iteration; ntile: 16-row tiles per wavefront. Shapes without an entry use DEFAULT_KERNEL.
+# iteration; ntile: 16-row tiles per wavefront. Shapes without an entry take w4_plan.decode's choice, DEFAULT_KERNEL where it
+# has none or the GPU has no table.
 # Keys (N, K, M[, "silu"], "norm") name the GEMV configuration of the fused add + RMSNorm prologue
 # (forward_norm), timed on its own; the plain key's entry is used where there is none.
 # Tables are keyed by device name and by gfx architecture; finalize() tries the name it is given,
@@ -253,7 +254,8 @@ class W4Linear(nn.Module):
         self.register_buffer("scales", torch.empty(in_features // group, out_features, dtype=torch.float16))
         self.kernels: dict[tuple, W4Kernel] = {}
         self.gemm_kernels: dict[tuple, tuple[tuple[int, W4Gemm | None], ...]] = {}
-        self.cus = 256  # of the layer's GPU, for the rule (finalize)
+        self.cus = 256  # of the layer's GPU, for the rules (finalize)
+        self.decode_rule = False  # w4_plan.decode for M <= 16 without an entry: on the GPUs that have a table
 
     def enable_silu_mul(self) -> bool:
         if not self.awq_layout or self.out_features % 16:
@@ -271,6 +273,7 @@ class W4Linear(nn.Module):
         self.register_buffer("zeros", zeros)
         self.awq_layout = False
         self.kernels = _table(W4_KERNELS, device_name, packed.device)
+        self.decode_rule = bool(self.kernels)
         self.gemm_kernels = _table(W4_GEMM_KERNELS, device_name, packed.device)
         self.cus = torch.cuda.get_device_properties(packed.device).multi_processor_count
         # device set-up and the split-K workspace now, not inside graph capture
@@ -322,17 +325,23 @@ class W4Linear(nn.Module):
         return f"{cfg[0]}{tuple(cfg[1:])}" if cfg[0] in ("mma", "tiled") else f"gemm{tuple(cfg)}"
 
     def decode_entry(self, m: int) -> W4Kernel:
-        """The table entry forward uses at 1 <= M <= 16."""
+        """The kernel forward uses at 1 <= M <= 16: the table's entry, else w4_plan's rule on the sizes."""
+        entry = self._table_entry(m)
+        if entry is None and self.decode_rule:
+            entry = w4_plan.decode(m, self.out_features, self.in_features, self.cus)
+        return entry or DEFAULT_KERNEL
+
+    def _table_entry(self, m: int) -> W4Kernel | None:
         key = (self.out_features, self.in_features, m)
-        return (self.kernels.get((*key, "silu")) if self.silu_mul else None) or self.kernels.get(key, DEFAULT_KERNEL)
+        return (self.kernels.get((*key, "silu")) if self.silu_mul else None) or self.kernels.get(key)
 
     def norm_entry(self, m: int) -> W4Kernel:
         """The entry forward_norm uses: (N, K, M[, "silu"], "norm") where the fused-norm GEMV was
         timed on its own and beats the plain entry plus a separate norm kernel (its best
         configuration differs from the plain GEMV's: qkv at M = 1 runs 5.2 us with (4, 4, 1) against
-        6.1 us with the plain table's (8, 2, 1)), else decode_entry."""
+        6.1 us with the plain table's (8, 2, 1)), else the plain table's entry."""
         key = (self.out_features, self.in_features, m) + (("silu",) if self.silu_mul else ()) + ("norm",)
-        return self.kernels.get(key) or self.decode_entry(m)
+        return self.kernels.get(key) or self._table_entry(m) or DEFAULT_KERNEL
 
     def forward_norm(self, x: torch.Tensor, residual: torch.Tensor | None, norm_weight: torch.Tensor,
                      eps: float) -> tuple[torch.Tensor, torch.Tensor]:
@@ -377,10 +386,7 @@ class W4Linear(nn.Module):
             ext = w4_hip.load()
             if ext is not None:
                 m = x.shape[0]
-                key = (self.out_features, self.in_features, m)
-                entry = (self.kernels.get((*key, "silu")) if self.silu_mul else None) or \
-                    self.kernels.get(key, DEFAULT_KERNEL)
-                kind, *cfg = entry
+                kind, *cfg = self.decode_entry(m)
                 if kind == "gemm":
                     return self._gemm(ext, x, cfg)
                 if kind == "gemv" and m <= 4:  # with the SwiGLU epilogue too (tw4_gemv_act)
