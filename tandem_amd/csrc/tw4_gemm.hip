@@ -602,10 +602,12 @@ int tw4_gemm_tiled_dispatch(const uint16_t* x, const int32_t* packed, const uint
 
 namespace {
 
-// The argument checks every GEMM entry point shares, and the device's set-up (index in dev).
+// The argument checks every GEMM entry point shares, and the device's set-up (index in dev). lds: the kernel with both
+// tiles in LDS, whose loads take per-lane byte offsets of 32 bits: x (2 M K bytes) and the packed weights, whose last row
+// tile is 16 rows also where N ends after 8 (padded N K / 2 bytes).
 int gemm_check(const uint16_t* x, const int32_t* packed, const uint16_t* scales, const uint16_t* zeros, const uint16_t* y,
                const float* ws, const int32_t* locks, int64_t ws_floats, int64_t n_locks, int M, int N, int K, int splits,
-               int act, int& dev) {
+               int act, bool lds, int& dev) {
     TW4_REQUIRE(x && packed && scales && zeros && y, TW4_EINVAL, "gemm: null pointer");
     TW4_REQUIRE(reinterpret_cast<uintptr_t>(x) % 16 == 0, TW4_EINVAL, "gemm: x must be 16-byte aligned");
     TW4_REQUIRE(reinterpret_cast<uintptr_t>(packed) % 16 == 0, TW4_EINVAL, "gemm: packed must be 16-byte aligned");
@@ -619,6 +621,8 @@ int gemm_check(const uint16_t* x, const int32_t* packed, const uint16_t* scales,
     TW4_REQUIRE(splits <= 1 || (ws && locks), TW4_EINVAL, "gemm: split-K needs a workspace and counters");
     TW4_REQUIRE(ws_floats >= 0 && n_locks >= 0, TW4_EINVAL, "gemm: workspace sizes must be >= 0");
     if (M == 0) return TW4_OK;
+    TW4_REQUIRE(!lds || (static_cast<int64_t>(M) * K < (1LL << 31) && ((N + 15LL) & ~15LL) * K < (1LL << 33)), TW4_EINVAL,
+                "gemm (both tiles in LDS): M K < 2^31 and padded N K < 2^33 (M %d, N %d, K %d)", M, N, K);
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return tw4host::hip_fail(e, "gemm: hipGetDevice");
     if (dev < 0 || dev >= kMaxDevices || !g_dev[dev].ready) return device_prepare(dev);
@@ -632,7 +636,7 @@ extern "C" int tw4_gemm_tiled(const uint16_t* x, const int32_t* packed, const ui
                               int K, int mt, int nt, int warps_n, int warps_m, int warps_k, int ring, int splits, int act,
                               void* stream) {
     int dev = 0;
-    const int rc = gemm_check(x, packed, scales, zeros, y, ws, locks, ws_floats, n_locks, M, N, K, splits, act, dev);
+    const int rc = gemm_check(x, packed, scales, zeros, y, ws, locks, ws_floats, n_locks, M, N, K, splits, act, true, dev);
     if (rc || M == 0) return rc;
     if (splits == 0 && !(ws && locks)) splits = 1;
     return tw4_gemm_tiled_dispatch(x, packed, scales, zeros, y, ws, locks,
@@ -645,7 +649,7 @@ extern "C" int tw4_gemm(const uint16_t* x, const int32_t* packed, const uint16_t
                         int K, int mt, int nt, int warps_n, int warps_k, int stages, int splits, int act,
                         void* stream) {
     int dev = 0;
-    const int rc = gemm_check(x, packed, scales, zeros, y, ws, locks, ws_floats, n_locks, M, N, K, splits, act, dev);
+    const int rc = gemm_check(x, packed, scales, zeros, y, ws, locks, ws_floats, n_locks, M, N, K, splits, act, stages == 3, dev);
     if (rc || M == 0) return rc;
     ws_floats = ws_floats < kMaxPartialFloats ? ws_floats : kMaxPartialFloats;  // the part split-K may use
     if (splits == 0 && !(ws && locks)) splits = 1;

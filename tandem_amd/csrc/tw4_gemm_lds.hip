@@ -392,9 +392,6 @@ template <class C>
 int lds_gemm_launch(const h1* x, const u4* w, const h1* s, const h1* z, h1* y, float* ws, int* locks,
                     int64_t ws_floats, int64_t n_locks, int M, int N, int K, int splits, int cus, int act,
                     hipStream_t stream) {
-    // the loads' per-lane byte offsets are 32-bit: x (M K 2 bytes) and the weights (N K / 2 bytes)
-    TW4_REQUIRE(static_cast<int64_t>(M) * K < (1LL << 31) && static_cast<int64_t>(N) * K < (1LL << 33), TW4_EINVAL,
-                "gemm (both tiles in LDS): M K < 2^31 and N K < 2^33 (M %d, N %d, K %d)", M, N, K);
     TW4_REQUIRE(reinterpret_cast<uintptr_t>(s) % 4 == 0 && reinterpret_cast<uintptr_t>(z) % 4 == 0, TW4_EINVAL,
                 "gemm (both tiles in LDS): scales and zeros must be 4-byte aligned");
     const int G = K >> 7, stages = 2 * G;

@@ -98,7 +98,7 @@ def choose(m: int, n: int, k: int, act: bool = False, cus: int = 256) -> tuple |
             return True
         return splits <= groups and tiles <= PARTIAL_COUNTERS and tiles * splits * tile_floats <= PARTIAL_FLOATS
 
-    if n * k < 1 << 33:
+    if 16 * _cdiv(n, 16) * k < 1 << 33:  # the tiled kernel's 32-bit weight offsets, over whole row tiles
         floor = 2.0 * m * n * k / (TILED_PFLOPS * 1e9)
         for c, (occ, t0, s_full, s_one, d0, d1, u1) in TILED.items():
             bm, bn = 16 * c[0] * c[3], 16 * c[1] * c[2]

@@ -58,6 +58,11 @@ def test_argument_errors_return_before_launch():
                        ({"n": 24, "act": 1}, "SwiGLU"), ({"splits": 17}, "splits"), ({"splits": 2, "ws": None}, "workspace")):
         assert call(**kw) == w4_hip.TW4_EINVAL
         assert needle in lib.tw4_last_error().decode(), (kw, lib.tw4_last_error())
+    # the packed weights end at a whole row tile: N = 8 mod 16 just under 2^33 / K passes 2^32 bytes with its padding rows
+    n, k = 1677720, 5120
+    assert n * k < 1 << 33 <= (n + 8) * k
+    assert call(n=n, k=k) == w4_hip.TW4_EINVAL and "2^33" in lib.tw4_last_error().decode()
+    assert all((w4_plan.choose(m, n, k) or ("",))[0] != "tiled" for m in (17, 300, 4096))
     assert call(m=0) == w4_hip.TW4_OK
     assert lib.tw4_capture_id(None) == 0
 
