@@ -40,7 +40,7 @@ import torch.nn.functional as F
 from torch import nn
 
 from tandem_amd.layers import w4_hip, w4_plan
-from tandem_amd.layers.w4_tables import GFX950_DECODE, GFX950_GEMM
+from tandem_amd.layers.w4_tables import GFX950_DECODE, GFX950_GEMM, OTHERS, RuleLadder
 
 # Nibble of an AutoAWQ word that holds feature j = 0..7 of its 8: the packer writes features
 # 0, 2, 4, 6, 1, 3, 5, 7 into nibbles 0..7, so feature j is found at this position
@@ -171,13 +171,14 @@ W4_KERNELS: dict[str, dict[tuple, W4Kernel]] = {
 # M > 16: measured ladders per GPU and (N, K) / (N, K, "silu"), ((m_max, config), ...) by increasing m_max. config =
 # (MT, NT, WARPS_N, WARPS_K, STAGES, SPLITS) of w4_gemm, ("mma", warps_k, unroll, ntile): the streaming matrix-core kernel
 # of the decode path, whose 16-token batch tiles cover M <= 64, ("tiled", MT, NT, WARPS_N, WARPS_M, WARPS_K, RING, SPLITS)
-# of w4_gemm_tiled, or None: dequantize to float16 + torch.matmul. Past a ladder's last m_max, and for shapes without
-# one, w4_plan.choose picks the kernel from the sizes (the built-in ladders end at M = 64: past it the rule's choice is
-# as fast as the measured rungs were, and faster wherever w4_gemm_tiled is). DEFAULT_GEMM is the ladder of shapes
-# without an entry: no rung.
+# of w4_gemm_tiled, or None: dequantize to float16 + torch.matmul. The built-in ladders are RuleLadders: past their last
+# m_max w4_plan.choose picks the kernel from the sizes, as it does from M = 17 on for the shapes they do not name (the table's
+# OTHERS entry). A ladder that a caller puts in their place keeps its own meaning (pick_gemm: past the last m_max, the
+# last entry). DEFAULT_GEMM is the ladder of a layer without a table, or whose table names neither the shape nor OTHERS.
 # TANDEM_W4_GEMM=0: always dequantize + torch.matmul (python/tandem/layers/awq.py:163-186).
 W4Gemm = tuple
-DEFAULT_GEMM: tuple[tuple[int, W4Gemm | None], ...] = ()
+DEFAULT_GEMM: tuple[tuple[int, W4Gemm | None], ...] = (
+    (64, ("mma", 8, 1, 1)), (1024, (4, 2, 4, 1, 2, 0)), (1 << 30, None))
 W4_GEMM_KERNELS: dict[str, dict[tuple, tuple[tuple[int, W4Gemm | None], ...]]] = {
     MI355X: GFX950_GEMM,
     GFX950: GFX950_GEMM,
@@ -299,11 +300,13 @@ class W4Linear(nn.Module):
         return call(x, self.packed, self.scales, self.zeros, buf, locks, *cfg, int(self.silu_mul))
 
     def gemm_entry(self, m: int, x: torch.Tensor | None = None) -> W4Gemm | None:
-        """The M > 16 kernel: the shape's ladder up to its last m_max, then w4_plan's rule on the sizes (for an x
+        """The M > 16 kernel: the shape's ladder, continued by w4_plan's rule on the sizes where it is a RuleLadder (for an x
         that autograd or a transform follows: None, dequantize + F.linear)."""
         key = (self.out_features, self.in_features) + (("silu",) if self.silu_mul else ())
-        ladder = self.gemm_kernels.get(key, DEFAULT_GEMM)
-        if ladder and m <= ladder[-1][0]:
+        ladder = self.gemm_kernels.get(key)
+        if ladder is None:
+            ladder = self.gemm_kernels.get(OTHERS, DEFAULT_GEMM)
+        if not isinstance(ladder, RuleLadder) or (ladder and m <= ladder[-1][0]):
             return pick_gemm(ladder, m)
         if x is not None and not w4_hip.plain(x):
             return None
