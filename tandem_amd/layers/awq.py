@@ -301,7 +301,8 @@ class W4Linear(nn.Module):
 
     def gemm_entry(self, m: int, x: torch.Tensor | None = None) -> W4Gemm | None:
         """The M > 16 kernel: the shape's ladder, continued by w4_plan's rule on the sizes where it is a RuleLadder (for an x
-        that autograd or a transform follows: None, dequantize + F.linear)."""
+        that autograd or a transform follows: None, dequantize + F.linear; where autocast, a mode or a compiler follows the
+        call: fused up to the ladder's fused_rows, None past them)."""
         key = (self.out_features, self.in_features) + (("silu",) if self.silu_mul else ())
         ladder = self.gemm_kernels.get(key)
         if ladder is None:
@@ -310,7 +311,10 @@ class W4Linear(nn.Module):
             return pick_gemm(ladder, m)
         if x is not None and not w4_hip.plain(x):
             return None
-        return w4_plan.choose(m, self.out_features, self.in_features, self.silu_mul, self.cus)
+        cfg = w4_plan.choose(m, self.out_features, self.in_features, self.silu_mul, self.cus)
+        if x is not None and w4_hip.intercepted():
+            return None if m > ladder.fused_rows else cfg or pick_gemm(DEFAULT_GEMM, min(m, 1024))
+        return cfg
 
     def kernel_for(self, m: int) -> str:
         """The kernel forward runs for a 16-byte aligned fp16 x of M rows on the GPU, by the same

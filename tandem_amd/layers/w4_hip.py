@@ -23,6 +23,8 @@ import threading
 
 import torch
 from torch.autograd import forward_ad
+from torch.overrides import _get_current_function_mode_stack
+from torch.utils._device import DeviceContext
 
 LIB_PATH = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "lib", "libtandem_w4.so")
 
@@ -470,12 +472,24 @@ def stream_workspace(device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
 
 def plain(x: torch.Tensor) -> bool:
     """An ordinary tensor that only the values of this call matter to: no gradient or tangent is asked of it, no transform
-    (vmap, jvp), tracer, compiler or dispatch mode follows the call. Anything else has to stay in torch operators, as a kernel that
+    (vmap, jvp), tracer or dispatch mode follows the call. Anything else has to stay in torch operators, as a kernel that
     sees a data pointer only would drop what follows it."""
     return (type(x) in (torch.Tensor, torch.nn.Parameter) and not (x.requires_grad and torch.is_grad_enabled())
-            and not torch.compiler.is_compiling() and not torch._C._is_tracing()
-            and not torch._C._len_torch_dispatch_stack() and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+            and not torch._C._is_tracing() and not torch._C._len_torch_dispatch_stack()
+            and not torch._C._functorch.is_functorch_wrapped_tensor(x)
             and (forward_ad._current_level < 0 or forward_ad.unpack_dual(x).tangent is None))
+
+
+def intercepted() -> bool:
+    """Whether a torch operator called here would come out otherwise than by its arguments: autocast to another type than
+    float16 gives a product another dtype, a torch function mode sees or replaces it (a default device does neither), a
+    compiler puts it into its graph. A call that was a torch operator stays one there; one that was a kernel stays a kernel."""
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.float16:
+        return True
+    if torch._C._len_torch_function_stack() and any(not isinstance(mode, DeviceContext)
+                                                    for mode in _get_current_function_mode_stack()):
+        return True
+    return torch.compiler.is_compiling()
 
 
 @functools.lru_cache(maxsize=None)

@@ -102,9 +102,9 @@ class Attention(nn.Module):
         self.o_proj = make_linear(self.q_size, cfg.hidden_size, False, quant)
 
     def _hip_attend(self, qkv: torch.Tensor) -> bool:
-        """Plain contiguous 16-byte aligned fp16 GPU rows [q | k | v] that no gradient or transform follows, whole 16-byte
-        chunks per head: tw4_attend_one; anything else the torch expression of the same copy."""
-        return (w4_hip.plain(qkv) and qkv.is_cuda and qkv.dtype == torch.float16 and qkv.dim() == 2 and qkv.numel() > 0
+        """Plain contiguous 16-byte aligned fp16 GPU rows [q | k | v] that no gradient, transform, mode or compiler follows, whole
+        16-byte chunks per head: tw4_attend_one; anything else the torch expression of the same copy."""
+        return (w4_hip.plain(qkv) and not w4_hip.intercepted() and qkv.is_cuda and qkv.dtype == torch.float16 and qkv.dim() == 2 and qkv.numel() > 0
                 and qkv.is_contiguous()
                 and qkv.shape[1] == self.q_size + 2 * self.kv_size and self.head_dim % 8 == 0
                 and self.num_heads % self.num_kv_heads == 0 and qkv.data_ptr() % 16 == 0

@@ -2,12 +2,20 @@
 
 from __future__ import annotations
 
+import contextlib
 import copy
+import ctypes
 import pickle
+import types
 
+import numpy as np
 import pytest
+import torch
+import torch.nn.functional as F
+from torch.overrides import TorchFunctionMode
 
-from tandem_amd.layers import awq, w4_plan
+from oracle import awq_oracle as o
+from tandem_amd.layers import awq, gemv16, w4_hip, w4_plan
 from tandem_amd.layers.w4_tables import GFX950_GEMM, OTHERS, RuleLadder
 
 FIXED = ((64, ("mma", 8, 1, 1)), (1024, (4, 2, 4, 1, 2, 0)), (1 << 30, None))
@@ -57,3 +65,96 @@ def test_ladders_survive_a_copy_of_the_layer():
         assert other.gemm_kernels == GFX950_GEMM
         for m in (17, 700, 5000):
             assert other.gemm_entry(m) == _layer().gemm_entry(m)
+        assert all(a.fused_rows == b.fused_rows for a, b in zip(other.gemm_kernels.values(), GFX950_GEMM.values()))
+
+
+@contextlib.contextmanager
+def _autocast(dtype):
+    """torch.autocast("cuda", dtype) without the check for a GPU."""
+    was = torch.is_autocast_enabled("cuda"), torch.get_autocast_dtype("cuda")
+    torch.set_autocast_enabled("cuda", True)
+    torch.set_autocast_dtype("cuda", dtype)
+    try:
+        yield
+    finally:
+        torch.set_autocast_enabled("cuda", was[0])
+        torch.set_autocast_dtype("cuda", was[1])
+
+
+class _Counting(TorchFunctionMode):
+    seen = 0
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.seen += func is F.linear
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("follow", [lambda: _autocast(torch.bfloat16), _Counting])
+def test_followed_calls_keep_their_side_of_f_linear(follow):
+    """Autocast decides the dtype of F.linear's result and a function mode sees the call: past fused_rows, where the layer
+    dequantized for F.linear before it had a rule, it does so there still, and below it stays a kernel of its own."""
+    for (k, n), rows in (((4096, 6144), 1 << 18), ((12288, 4096), 2048), ((2048, 2048), 1024), ((2304, 4112), 1024)):
+        layer = _layer(k, n)
+        for m in (17, 300, 1024, 1025, 2048, 2049, 5000):
+            x = torch.empty(m, k, dtype=torch.float16)
+            assert layer.gemm_entry(m, x) == layer.gemm_entry(m)
+            with follow():
+                e = layer.gemm_entry(m, x)
+                assert (e is None) == (m > rows), (k, n, m, e)
+    with _autocast(torch.float16), torch.device("cpu"):  # neither changes a product of float16 tensors
+        assert not w4_hip.intercepted() and layer.gemm_entry(5000, x) == layer.gemm_entry(5000)
+
+
+def test_compiled_layers_run_the_kernels(monkeypatch):
+    """Under torch.compile the launch is a graph break; the route is the eager one (dequantize + F.linear past fused_rows)."""
+    calls = []
+    native = ctypes.CDLL(None).labs  # as a launch: nothing a compiler can trace
+
+    def kernel(name):
+        def run(x, *args):
+            native(ctypes.c_long(x.data_ptr()))
+            calls.append(name)
+            return x[:, :64] * 1
+        return run
+
+    ext = types.SimpleNamespace(w4_mma=kernel("kernel"), w4_gemm=kernel("kernel"), w4_gemm_tiled=kernel("kernel"))
+    monkeypatch.setattr(awq, "_gemm_ok", lambda x: x.shape[0] > 16)
+    monkeypatch.setattr(awq, "_hip_ok", lambda x: x.shape[0] <= 16)
+    monkeypatch.setattr(w4_hip, "load", lambda: ext)
+    for name in ("workspace", "stream_workspace"):
+        monkeypatch.setattr(w4_hip, name, lambda device: (None, None))
+    monkeypatch.setattr(awq.W4Linear, "_dense", lambda self, x: (calls.append("dense"), x[:, :64] * 1)[1])
+    layer = _layer(256, 64)
+    layer.packed = layer.zeros = None
+    torch._dynamo.reset()
+    compiled = torch.compile(layer, backend="eager")
+    for m, want in ((17, "kernel"), (100, "kernel"), (1024, "kernel"), (1025, "dense")):
+        calls.clear()
+        compiled(torch.zeros(m, 256, dtype=torch.float16))
+        assert calls == [want], (m, calls)
+    torch._dynamo.reset()
+
+
+@pytest.mark.gpu
+def test_autocast_and_modes_on_the_gpu():
+    raw = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in o.random_awq(1152, 1032, seed=3)[:3]]
+    layer = awq.W4Linear(1152, 1032, 128).cuda()
+    for name, t in zip(("qweight", "qzeros", "scales"), raw):
+        getattr(layer, name).copy_(t)
+    layer.finalize(torch.cuda.get_device_name())
+    w = torch.randn(32776, 2048, device="cuda", dtype=torch.float16) * 0.02
+    table = gemv16.table_for(torch.device("cuda"), torch.nn.Module())
+    x, xh = torch.randn(1100, 1152, device="cuda").half(), torch.randn(32, 2048, device="cuda").half()
+    plain, head = layer(x), gemv16.linear(xh, w, table)
+    dense, torch_head = F.linear(x, awq.w4_dequant(layer.packed, layer.scales, layer.zeros)), F.linear(xh, w)
+    for a, b in ((plain, dense), (head, torch_head)):
+        assert a.dtype == torch.float16
+        torch.testing.assert_close(a, b, rtol=2e-3, atol=2e-3)  # two roundings to fp16, sums in two orders
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert layer(x).dtype == gemv16.linear(xh, w, table).dtype == torch.bfloat16
+        assert layer(x[:300]).dtype == torch.float16
+    with _Counting() as mode:
+        assert torch.equal(layer(x), dense) and torch.equal(gemv16.linear(xh, w, table), torch_head)
+        assert mode.seen == 2
+        layer(x[:300])
+        assert mode.seen == 2
