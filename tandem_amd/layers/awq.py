@@ -237,7 +237,8 @@ class W4Linear(nn.Module):
     ``finalize`` replaces the three buffers by the tile layout (``packed``, ``scales``, ``zeros``) in
     one repack kernel and picks the device's kernel tables. From then on ``forward`` dispatches by
     batch size: the (N, K, M) decode table up to M = 16, the M > 16 ladder above, dequantize +
-    torch.matmul where the table says None, the switch is off or x is not 16-byte aligned.
+    torch.matmul where the table says None, the switch is off, x is not 16-byte aligned or, past M = 16, autograd or a
+    transform follows x (the decode kernels return a result that autograd does not follow).
 
     A SwiGLU MLP's gate_up calls ``enable_silu_mul`` before ``finalize``: the repack then interleaves
     gate and up rows by 8 and every kernel's epilogue returns silu(gate) * up, [M, out_features / 2]."""
@@ -300,17 +301,17 @@ class W4Linear(nn.Module):
         return call(x, self.packed, self.scales, self.zeros, buf, locks, *cfg, int(self.silu_mul))
 
     def gemm_entry(self, m: int, x: torch.Tensor | None = None) -> W4Gemm | None:
-        """The M > 16 kernel: the shape's ladder, continued by w4_plan's rule on the sizes where it is a RuleLadder (for an x
-        that autograd or a transform follows: None, dequantize + F.linear; where autocast, a mode or a compiler follows the
-        call: fused up to the ladder's fused_rows, None past them)."""
+        """The M > 16 kernel: the shape's ladder, continued by w4_plan's rule on the sizes where it is a RuleLadder (where
+        autocast, a mode or a compiler follows the call: fused up to the ladder's fused_rows, None past them). For an x that
+        autograd or a transform follows: None, dequantize + F.linear, which keeps the gradient of x at every M > 16."""
+        if x is not None and not w4_hip.plain(x):
+            return None
         key = (self.out_features, self.in_features) + (("silu",) if self.silu_mul else ())
         ladder = self.gemm_kernels.get(key)
         if ladder is None:
             ladder = self.gemm_kernels.get(OTHERS, DEFAULT_GEMM)
         if not isinstance(ladder, RuleLadder) or (ladder and m <= ladder[-1][0]):
             return pick_gemm(ladder, m)
-        if x is not None and not w4_hip.plain(x):
-            return None
         cfg = w4_plan.choose(m, self.out_features, self.in_features, self.silu_mul, self.cus)
         if x is not None and w4_hip.intercepted():
             return None if m > ladder.fused_rows else cfg or pick_gemm(DEFAULT_GEMM, min(m, 1024))

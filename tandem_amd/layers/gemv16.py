@@ -170,6 +170,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, table: dict[tuple[int, int, int], C
     M = 4, whose x the vector form keeps in LDS whole, tw4_gemv_f16 where it takes K: 184 us against 197 on the Qwen3-8B
     head at M = 1), through F.linear (hipBLASLt) otherwise (python/tandem/layers/triton_gemv.py:285-297)."""
     cfg = entry(x, w, table, eager)
+    if cfg is not None and not (w4_hip.plain(x) and w4_hip.plain(w)):
+        return F.linear(x, w)  # a gradient or a transform follows the call
     # F.linear's own result where autocast, a mode or a compiler would change it; a shape the table names stays a kernel up to
     # its last bucket
     named = x.dim() == 2 and x.shape[0] <= BUCKETS[-1] and (*w.shape, 4) in table

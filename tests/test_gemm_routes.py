@@ -158,3 +158,38 @@ def test_autocast_and_modes_on_the_gpu():
         assert mode.seen == 2
         layer(x[:300])
         assert mode.seen == 2
+
+
+@pytest.mark.parametrize("k,n", [(4096, 6144), (2304, 4112)])
+def test_an_x_that_autograd_follows_takes_no_kernel(k, n):
+    """Below a ladder's last m_max as past it."""
+    layer = _layer(k, n)
+    for m in (17, 24, 64, 65, 300, 5000):
+        x = torch.empty(m, k, dtype=torch.float16, requires_grad=True)
+        assert layer.gemm_entry(m, x) is None
+        with torch.no_grad():
+            assert layer.gemm_entry(m, x) == layer.gemm_entry(m)
+
+
+@pytest.mark.gpu
+def test_gradients_are_kept_at_every_size():
+    k, n = 4096, 6144  # a shape with a ladder
+    raw = [torch.from_numpy(np.ascontiguousarray(a)).cuda() for a in o.random_awq(k, n, seed=5)[:3]]
+    layer = awq.W4Linear(k, n, 128).cuda()
+    for name, t in zip(("qweight", "qzeros", "scales"), raw):
+        getattr(layer, name).copy_(t)
+    layer.finalize(torch.cuda.get_device_name())
+    w = awq.w4_dequant(layer.packed, layer.scales, layer.zeros)
+    for m in (24, 100):
+        x = torch.randn(m, k, device="cuda").half().requires_grad_()
+        layer(x).sum().backward()
+        assert torch.equal(x.grad, torch.autograd.grad(F.linear(x, w).sum(), x)[0])
+    head = torch.randn(151936, 2048, device="cuda", dtype=torch.float16) * 0.02
+    table = gemv16.table_for(torch.device("cuda"), torch.nn.Module())
+    assert (151936, 2048, 1) in table
+    for m in (1, 4, 8):
+        x = torch.randn(m, 2048, device="cuda").half().requires_grad_()
+        gemv16.linear(x, head, table).sum().backward()
+        assert torch.equal(x.grad, torch.autograd.grad(F.linear(x, head).sum(), x)[0])
+        assert gemv16.linear(x.detach(), head.requires_grad_(), table).requires_grad
+        head.requires_grad_(False)
