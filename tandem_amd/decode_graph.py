@@ -2,8 +2,9 @@
 
 A decode step with b sequences replays the graph of the smallest bucket >= b (1, 2, 4, 8, 16, 24,
 ... up to max_bs). Graphs are captured from the largest bucket down into one shared memory pool,
-after two eager warm-up passes on a side stream (the warm-up also allocates the split-K workspace
-and sets up the kernels, which must not happen inside a capture). Per step, outside the graph, the
+after two eager warm-up passes on a side stream, one for all buckets (the warm-up also sets up the
+kernels, which must not happen inside a capture; the decode kernels' split-K workspace is there since
+finalize, a bucket past 16 whose projections split K takes one from the graphs' own pool). Per step, outside the graph, the
 token ids are copied into the static input buffer (padding rows take token 0 and are computed but
 never returned); then the bucket's graph replays and the first b rows of its output are returned.
 
@@ -20,6 +21,8 @@ from typing import Callable, Sequence
 
 import torch
 from torch import nn
+
+from tandem_amd.layers import w4_hip
 
 logger = logging.getLogger(__name__)
 
@@ -57,9 +60,9 @@ class DecodeGraphRunner:
     @torch.inference_mode()
     def _capture_all(self) -> None:
         pool = torch.cuda.graph_pool_handle()
+        stream = torch.cuda.Stream(self.device)
         for bs in reversed(self.sizes):
             run = self._fn(bs)
-            stream = torch.cuda.Stream(self.device)
             stream.wait_stream(torch.cuda.current_stream(self.device))
             with torch.cuda.stream(stream):
                 for _ in range(2):
@@ -69,6 +72,7 @@ class DecodeGraphRunner:
             with torch.cuda.graph(graph, pool=pool):
                 self.outputs[bs] = run()
             self.graphs[bs] = graph
+        w4_hip.release_stream_workspace(stream)
         torch.cuda.synchronize(self.device)
         logger.info("captured HIP graphs for decode batch sizes %s", self.sizes)
 

@@ -281,7 +281,6 @@ class W4Linear(nn.Module):
         # device set-up and the split-K workspace now, not inside graph capture
         if w4_hip.load() is not None:
             w4_hip.workspace(packed.device)
-            w4_hip.stream_workspace(packed.device)
 
     def _dense(self, x: torch.Tensor) -> torch.Tensor:
         """HIP dequantize (gate_up: back in [gate | up] row order) + torch.matmul, and the same
@@ -293,8 +292,10 @@ class W4Linear(nn.Module):
         return silu_and_mul(y) if self.silu_mul else y
 
     def _gemm(self, ext, x: torch.Tensor, cfg) -> torch.Tensor:
-        # decode calls (M <= 16, captured with the workspace finalize made) use the device's, larger ones their stream's
-        buf, locks = w4_hip.workspace(x.device) if x.shape[0] <= 16 else w4_hip.stream_workspace(x.device)
+        # decode calls (M <= 16, captured with the workspace finalize made) use the device's, larger ones their stream's where
+        # they may split K (splits, the last number, 0: the library decides); an unsplit call writes to none
+        own = x.shape[0] > 16 and cfg[-1] != 1
+        buf, locks = w4_hip.stream_workspace(x.device) if own else w4_hip.workspace(x.device)
         call = ext.w4_gemm
         if cfg[0] == "tiled":
             call, cfg = ext.w4_gemm_tiled, cfg[1:]

@@ -15,6 +15,7 @@ act)``; each allocates y with torch on x's device and launches on the current st
 
 from __future__ import annotations
 
+import collections
 import contextlib
 import ctypes
 import functools
@@ -33,8 +34,8 @@ TW4_OK, TW4_EINVAL, TW4_ECONFIG, TW4_EHIP, TW4_ESPACE = 0, 1, 2, 3, 4
 WORKSPACE_FLOATS = 1 << 23  # 32 MB of float32 split-K partial sums per GPU (w4_cuda.py:24)
 WORKSPACE_LOCKS = 1 << 15
 _workspaces: dict[int, tuple[torch.Tensor, torch.Tensor]] = {}
-STREAM_WORKSPACES = 8  # at most this many per-stream workspaces are kept, the oldest given back first
-_stream_workspaces: dict[tuple[int, int, int], tuple[torch.Tensor, torch.Tensor]] = {}
+STREAM_WORKSPACES = 8  # at most this many per-stream workspaces are kept
+_stream_workspaces: collections.OrderedDict[tuple[int, int, int], tuple[torch.Tensor, torch.Tensor]] = collections.OrderedDict()
 _init_lock = threading.Lock()
 _initialized: set[int] = set()
 
@@ -441,33 +442,49 @@ def workspace(device: torch.device | str | int) -> tuple[torch.Tensor, torch.Ten
     index = dev.index if dev.index is not None else torch.cuda.current_device()
     buf = _workspaces.get(index)
     if buf is None:
-        dev = torch.device("cuda", index)
-        buf = (torch.empty(WORKSPACE_FLOATS, dtype=torch.float32, device=dev),
-               torch.zeros(WORKSPACE_LOCKS, dtype=torch.int32, device=dev))
-        _workspaces[index] = buf
+        buf = _workspaces[index] = _new_workspace(index)
     return buf
+
+
+def _new_workspace(index: int) -> tuple[torch.Tensor, torch.Tensor]:
+    dev = torch.device("cuda", index)
+    return (torch.empty(WORKSPACE_FLOATS, dtype=torch.float32, device=dev),
+            torch.zeros(WORKSPACE_LOCKS, dtype=torch.int32, device=dev))
 
 
 def stream_workspace(device: torch.device) -> tuple[torch.Tensor, torch.Tensor]:
     """``workspace`` for the current stream alone, so calls on several streams (or threads with a stream each) and
-    graphs replayed side by side share no partial sums: one per stream, and one per graph capture, which takes it from
-    the graph's own memory and clears its counters there. A buffer given back returns to its stream's (its graph's) pool,
-    where whatever takes it next is ordered behind the kernels that used it."""
+    graphs replayed side by side share no partial sums: one per stream, and one per graph capture and stream in it, which
+    takes it from the graph's own memory and clears its counters there. STREAM_WORKSPACES are kept, the least recently used
+    one is given back (more streams in turn than that make one anew at each call), and those of an earlier capture at the
+    next one. A buffer given back returns to its stream's (its graph's) pool, where whatever takes it next is ordered behind
+    the kernels that used it."""
     index = device.index if device.index is not None else torch.cuda.current_device()
     stream = raw_stream(index)
     capture = library().tw4_capture_id(stream) if stream else 0
     key = (index, stream, capture)
-    buf = _stream_workspaces.get(key)
-    if buf is None:
-        with _init_lock:
-            for old in [k for k in _stream_workspaces if capture and k[2]]:  # one capture's at a time
-                del _stream_workspaces[old]
-            while len(_stream_workspaces) >= STREAM_WORKSPACES:
-                del _stream_workspaces[next(iter(_stream_workspaces))]
-            dev = torch.device("cuda", index)
-            buf = _stream_workspaces[key] = (torch.empty(WORKSPACE_FLOATS, dtype=torch.float32, device=dev),
-                                             torch.zeros(WORKSPACE_LOCKS, dtype=torch.int32, device=dev))
+    try:
+        _stream_workspaces.move_to_end(key)
+        return _stream_workspaces[key]
+    except KeyError:  # none yet, or given back by another thread just now
+        pass
+    with _init_lock:
+        for old in list(_stream_workspaces):
+            if capture and old[2] not in (0, capture):
+                _stream_workspaces.pop(old, None)
+        while len(_stream_workspaces) >= STREAM_WORKSPACES:
+            _stream_workspaces.popitem(last=False)
+        buf = _stream_workspaces[key] = _new_workspace(index)
     return buf
+
+
+def release_stream_workspace(stream: torch.cuda.Stream) -> None:
+    """Give back what stream_workspace keeps for a stream that is done with (a warm-up's) and for graph captures. A later call
+    there makes its own again."""
+    with _init_lock:
+        for key in list(_stream_workspaces):
+            if key[:2] == (stream.device_index, stream.cuda_stream) or key[2]:
+                _stream_workspaces.pop(key, None)
 
 
 def plain(x: torch.Tensor) -> bool:
