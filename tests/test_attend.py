@@ -35,7 +35,10 @@ def test_attend_matches_torch(m, heads, kv, dim):
     for x in (qkv.cuda(), flat[1:].view(qkv.shape), wide[:, :qkv.shape[1]], qkv.float().cuda()):
         y = attn.attend(x)
         assert y.is_contiguous() and y.dtype == x.dtype and torch.equal(y.half().cpu(), want)
-    x = qkv.cuda().requires_grad_()
+    x = qkv.cuda()
+    copies = attn.attend(x).untyped_storage().data_ptr() != x.untyped_storage().data_ptr()
+    assert m == 0 or copies == (m > 1 or heads > kv)  # one row of as many KV heads: a view
+    x.requires_grad_()
     attn.attend(x).float().sum().backward()
     assert float(x.grad.double().sum()) == m * heads * dim
 
