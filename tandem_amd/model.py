@@ -107,7 +107,8 @@ class Attention(nn.Module):
         head for each query head is no copy at all: its value columns as they lie."""
         return (w4_hip.plain(qkv) and not w4_hip.intercepted() and qkv.is_cuda and qkv.dtype == torch.float16
                 and qkv.dim() == 2 and qkv.numel() > 0 and qkv.is_contiguous()
-                and not (qkv.shape[0] == 1 and self.num_heads == self.num_kv_heads) and qkv.shape[1] == self.q_size + 2 * self.kv_size and self.head_dim % 8 == 0
+                and not (qkv.shape[0] == 1 and self.num_heads == self.num_kv_heads)
+                and qkv.shape[1] == self.q_size + 2 * self.kv_size and self.head_dim % 8 == 0
                 and self.num_heads % self.num_kv_heads == 0 and qkv.data_ptr() % 16 == 0
                 and 8 * (1 << 31) > qkv.numel())
 
