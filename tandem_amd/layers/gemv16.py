@@ -1,13 +1,14 @@
-"""Small-batch fp16 GEMV for decode on MI355X: y[M, N] = x[M, K] @ w[N, K]^T, M <= 8.
+"""Small-batch fp16 products for decode on MI355X: y[M, N] = x[M, K] @ w[N, K]^T, M <= 32.
 
 Drop-in for python/tandem/layers/triton_gemv.py (12vivi/tandem) on the path of a W4A16 model's
 fp16 lm_head: the same ``gemv`` / ``linear`` / ``install`` / ``table_for`` / ``default_table``
 functions, the same per-GPU ``CONFIGS`` keyed by (N, K, M bucket) and the same fallback to
-``F.linear`` (hipBLASLt here) for shapes without an entry. The kernel is tw4_gemv_f16 of
-libtandem_w4.so (hand-written HIP for gfx950, no Triton): it streams every row of w once with
-coalesced 16-byte loads and reduces on v_dot2_f32_f16, so it is bound by HBM bandwidth; for the
-M = 8 bucket a matrix-core form (config rows_inflight 16 or 32) multiplies 16-row tiles of w with x
-on v_mfma_f32_16x16x32_f16 instead, which reads x from LDS once per 16 rows rather than once per row.
+``F.linear`` (hipBLASLt here). Two kernels of libtandem_w4.so (hand-written HIP for gfx950, no
+Triton), both bound by streaming w once: tw4_gemv_f16 (``gemv``, M <= 8, a config from the table) with
+coalesced 16-byte loads and v_dot2_f32_f16, and tw4_gemm_f16 (``gemm``, M <= 32) on the matrix cores with
+both operands through LDS, which ``linear`` takes by a rule on sizes (``streams``) for the shapes and batches
+the table does not name. A matrix-core form of tw4_gemv_f16 (rows_inflight 16 or 32) stays as a
+configuration a caller's table can name; no built-in entry does (tw4_gemm_f16 is faster).
 
 The reference's fused norm / activation prologue (triton_gemv.py:92-178, 330-415) is not part of
 this build: it enabled no shape there (triton_gemv.py:316-329).
@@ -27,7 +28,7 @@ from tandem_amd.layers import w4_hip
 # 16 / 32: the matrix-core form with one / two 128-k chunks per step in flight, rows_per_wave a
 # multiple of 16), the fastest of
 # `python bench.py tune --projs lm_head --kinds dense16,torch16` on the GPU. Shapes without
-# an entry keep F.linear (python/tandem/layers/triton_gemv.py:221-268). Keyed by device name and by
+# an entry take ``streams``' rule, else F.linear (python/tandem/layers/triton_gemv.py:221-268). Keyed by device name and by
 # gfx architecture.
 Config = tuple[int, int]
 GFX950_DENSE: dict[tuple[int, int, int], Config] = {
@@ -138,25 +139,31 @@ def gemm(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return out
 
 
-# Where tw4_gemm_f16 (and tw4_gemv_f16 up to M = 4) takes a product no table entry names: weights of at least this many
-# bytes and at most 32 rows. Against F.linear (hipBLASLt) on MI355X, us: 1.24 GB (4096 x 151936) 197 / 212 / 221 at M = 8 / 24
-# / 32 against 248 / 260 / 265, 0.78 GB (2560 wide) 120 / 136 / 148 against 244 / 166 / 168, 134 MB (4096 x 16384) 28.6-29.5
-# against 32; at 67 MB (4096 x 8192, 2048 x 16384) launch and first loads decide and hipBLASLt is ahead (22 against 15,
-# 16.3 against 15.0), and at 48 rows x from L2 makes it level (250 against 252).
+# Where tw4_gemm_f16 (and tw4_gemv_f16 up to M = 4) takes a product no table entry names: at most 32 rows, at least
+# this many bytes of weights, and enough output columns. Against F.linear (hipBLASLt) on MI355X, us: 1.24 GB (4096 x
+# 151936) 197 / 212 / 221 at M = 8 / 24 / 32 against 248 / 260 / 265, 0.78 GB (2560 wide) 120 / 136 / 148 against 244 / 166 / 168,
+# 134 MB (4096 x 16384) 28.6-29.5 against 32; at 67 MB (4096 x 8192, 2048 x 16384) launch and first loads decide and hipBLASLt is
+# ahead (22 against 15, 16.3 against 15.0), and at 48 rows x from L2 makes it level (250 against 252).
+# Columns: the kernel deals 16-row tiles of w to two workgroups per CU and never splits K. Below about two passes of 64 rows
+# per CU most of the GPU idles: 8192 x 8192 40 us against 30, 16384 x 4096 45 against 30, 5120 x 16384 1.00-1.11 of hipBLASLt's
+# time at M = 16-32. Over 14 K from 1024 to 28672 x 11 N x 10 M: from N = 20480 on 0.30-1.03 of it, at N = 16384 up to
+# K = 4160 0.62-0.92; the rows of x, read from L2 for every 64 of w, pass it at M > 24 and K = 12288 (49152 columns 1.05).
 GEMM_MIN_BYTES = 128 << 20
 GEMM_MAX_ROWS = 32
 
 
+def streams(m: int, n: int, k: int) -> bool:
+    """Whether tw4_gemm_f16 is the faster kernel for m rows and n x k weights (see above), and takes the sizes."""
+    return (1 <= m <= GEMM_MAX_ROWS and k % 64 == 0 and GEMM_MIN_BYTES <= 2 * n * k < 1 << 32
+            and (n >= 20480 or (n >= 16384 and k <= 4160)) and (m <= 24 or k <= 8192))
+
+
 def _streams(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether F.linear(x, w) is a product bound by streaming w that tw4_gemm_f16 takes: up to
-    GEMM_MAX_ROWS rows, at least GEMM_MIN_BYTES of weights (and N K < 2^31), K a multiple of 64, plain contiguous aligned
-    float16 GPU tensors that no gradient or transform follows."""
-    if x.dim() != 2 or w.dim() != 2 or not 1 <= x.shape[0] <= GEMM_MAX_ROWS:
+    """Whether F.linear(x, w) is a product bound by streaming w that tw4_gemm_f16 takes: sizes that ``streams``, plain
+    contiguous aligned float16 GPU tensors that no gradient or transform follows."""
+    if x.dim() != 2 or w.dim() != 2 or x.shape[1] != w.shape[1] or not streams(x.shape[0], *w.shape):
         return False
-    if x.dtype != torch.float16 or w.dtype != torch.float16:
-        return False
-    n, k = w.shape
-    if k % 64 or x.shape[1] != k or not GEMM_MIN_BYTES <= 2 * n * k < 1 << 32 or not x.is_cuda or w.device != x.device:
+    if x.dtype != torch.float16 or w.dtype != torch.float16 or not x.is_cuda or w.device != x.device:
         return False
     if not (w4_hip.plain(x) and w4_hip.plain(w) and x.is_contiguous() and w.is_contiguous()):
         return False
@@ -178,7 +185,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, table: dict[tuple[int, int, int], C
     if cfg is None and eager and table and _streams(x, w) and (named or not w4_hip.intercepted()):
         if x.shape[0] > 4 or x.shape[1] not in KS:
             return gemm(x, w)
-        cfg = (2, 32) if w.shape[0] >= 1 << 16 else (2, 16)  # rows per wavefront: enough wavefronts for the GPU
+        # rows per wavefront: 32 for the long rows of K = 4096 (20480 columns 0.49 against 0.59 of F.linear's time at M = 1),
+        # 16 for shorter ones and few columns, where they leave wavefronts short (1024 x 102400 at M = 4 1.06 against 0.92)
+        cfg = (2, 32) if w.shape[1] > 2048 and w.shape[0] >= 20480 else (2, 16)
     return F.linear(x, w) if cfg is None else gemv(x, w, *cfg)
 
 

@@ -45,6 +45,16 @@ def test_gemm_tile_edges(m, n, k):
     _check(gemv16.gemm(x, w), x, w)
 
 
+def test_few_columns_stay_with_the_library():
+    """Where the kernel's 64-row passes leave most CUs idle or x outgrows L2, F.linear is the faster one (up to 2x)."""
+    for n, k in ((1024, 65536), (2048, 32768), (4736, 14336), (8192, 8192), (12288, 8192), (16384, 8192), (8192, 28672)):
+        assert 2 * n * k >= gemv16.GEMM_MIN_BYTES and not any(gemv16.streams(m, n, k) for m in (1, 5, 17, 32))
+    for n, k in ((131080, 512), (65536, 1024), (32776, 2048), (16384, 4096), (32000, 5120), (128256, 8192), (151936, 2560)):
+        assert all(gemv16.streams(m, n, k) for m in (1, 5, 17, 32)) and not gemv16.streams(33, n, k)
+    assert gemv16.streams(24, 49152, 12288) and not gemv16.streams(32, 49152, 12288)
+    assert not gemv16.streams(8, 32768, 4000) and not gemv16.streams(8, 1 << 20, 2048) and not gemv16.streams(0, 32776, 2048)
+
+
 @pytest.mark.gpu
 def test_linear_takes_it_where_streaming_w_bounds(monkeypatch):
     table = gemv16.table_for(torch.device("cuda"), torch.nn.Module())
