@@ -229,13 +229,14 @@ __device__ __forceinline__ int xcd_remap(int b, int n) {
 // atomics on gfx950 (the compiler's relaxed agent-scope load / store): they are coherent across
 // the XCDs' L2s without a cache-wide write-back or invalidate. s_waitcnt vmcnt(0) + barrier order
 // the stores before the count; the last arriver issues its loads only after it has seen the count
-// reach nsplit. The last arriver loads the partials of VB splits at a time (one memory round trip
-// per VB splits) and adds them in split order. act = 1: SwiGLU epilogue (gate rows 4 kb + i and up
+// reach nsplit. The last arriver loads FC fragments of VB splits at a time (one memory round trip
+// per VB splits) and adds them in split order. FRAGS: fragments per round, fewer than a wavefront's
+// where its sums alone fill half the registers it may have. act = 1: SwiGLU epilogue (gate rows 4 kb + i and up
 // rows 8 + 4 kb + i sit in lanes l and l + 32).
 constexpr int kCoherentAux = 16;  // buffer-instruction cache policy: sc1
 constexpr int64_t kMaxPartialFloats = int64_t(1) << 29;  // split-K workspace used: byte offsets < 2^31
 
-template <int MT, int NT, int WN, int PART_FLOATS = 64>
+template <int MT, int NT, int WN, int PART_FLOATS = 64, int FRAGS = MT * NT>
 __device__ __forceinline__ void finish_unit(f4 (&acc)[NT][MT], bool holder, int wn, int lane, int tid, int nsplit,
                                             int st, int su, float* __restrict__ ws, int* __restrict__ locks,
                                             int& last_flag, h1* __restrict__ y, int M, int N, int m0, int wt0,
@@ -263,30 +264,32 @@ __device__ __forceinline__ void finish_unit(f4 (&acc)[NT][MT], bool holder, int 
         __syncthreads();
         if (!last_flag) return;
         if (holder) {
-            constexpr int F = NT * MT;                        // 16-byte fragments per lane of one partial
-            constexpr int VB = 4 * F >= PART_FLOATS ? 1 : PART_FLOATS / (4 * F);  // splits per round
+            constexpr int F = NT * MT;  // 16-byte fragments per lane of one partial, FC of them at a time
+            constexpr int FC = F % FRAGS == 0 ? FRAGS : F;
+            constexpr int VB = 4 * FC >= PART_FLOATS ? 1 : PART_FLOATS / (4 * FC);  // splits per round
 #pragma unroll
             for (int t = 0; t < NT; ++t)
 #pragma unroll
                 for (int b = 0; b < MT; ++b) acc[t][b] = f4{0.0f, 0.0f, 0.0f, 0.0f};
-            for (int v0 = 0; v0 < nsplit; v0 += VB) {
-                f4 part[VB][F];
 #pragma unroll
-                for (int j = 0; j < VB; ++j) {
-                    const int v = min(v0 + j, nsplit - 1);  // past the last split: re-read it, not added
-                    const int other = static_cast<int>(((static_cast<int64_t>(st) * nsplit + v) * WN + wn) * V * 4);
+            for (int i0 = 0; i0 < F; i0 += FC) {
+                for (int v0 = 0; v0 < nsplit; v0 += VB) {
+                    f4 part[VB][FC];
 #pragma unroll
-                    for (int i = 0; i < F; ++i)
-                        part[j][i] = bitcast<f4>(__builtin_amdgcn_raw_buffer_load_b128(rs, (i * 64 + lane) * 16, other,
-                                                                                       kCoherentAux));
-                }
+                    for (int j = 0; j < VB; ++j) {
+                        const int v = min(v0 + j, nsplit - 1);  // past the last split: re-read it, not added
+                        const int other = static_cast<int>(((static_cast<int64_t>(st) * nsplit + v) * WN + wn) * V * 4);
 #pragma unroll
-                for (int j = 0; j < VB; ++j) {
-                    if (v0 + j >= nsplit) break;  // uniform
+                        for (int i = 0; i < FC; ++i)
+                            part[j][i] = bitcast<f4>(__builtin_amdgcn_raw_buffer_load_b128(
+                                rs, ((i0 + i) * 64 + lane) * 16, other, kCoherentAux));
+                    }
 #pragma unroll
-                    for (int t = 0; t < NT; ++t)
+                    for (int j = 0; j < VB; ++j) {
+                        if (v0 + j >= nsplit) break;  // uniform
 #pragma unroll
-                        for (int b = 0; b < MT; ++b) acc[t][b] += part[j][t * MT + b];
+                        for (int i = 0; i < FC; ++i) acc[(i0 + i) / MT][(i0 + i) % MT] += part[j][i];
+                    }
                 }
             }
         }

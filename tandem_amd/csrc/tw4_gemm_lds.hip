@@ -91,6 +91,10 @@ struct LdsGemmCfg {
     // wavefronts per SIMD the registers are kept for: two where the accumulators leave room for it and two
     // workgroups fit a CU's 160 KB of LDS (or the workgroup itself has eight wavefronts)
     static constexpr int MIN_WAVES_PER_SIMD = MT * NT <= 32 && (WAVES >= 8 || LDS_BYTES <= 80 * 1024 - 256) ? 2 : 1;
+    // partial sums the last arriver of a K split loads per round (finish_unit): all of a wavefront's, unless they and the sums
+    // they are added to fill every register, which left the compiler two loads in flight (128 x 256, 4096 x 4096 in 16
+    // splits: 90 us; half of them per round 42)
+    static constexpr int FRAGS = MT * NT == 64 || (MT * NT == 32 && MIN_WAVES_PER_SIMD == 2) ? MT * NT / 2 : MT * NT;
     static_assert(WK == 1 || (WK == 2 && WM * WN * MT * NT * 64 <= R * SLOT_U4), "the K halves' sums fit the ring");
     static_assert(R >= 3, "ring of at least 3 slots");
     static_assert(BM % 8 == 0 && BN % 32 == 0, "whole 1 KB loads");
@@ -377,7 +381,7 @@ gemm_lds_kernel(const h1* __restrict__ x, const u4* __restrict__ w, const h1* __
                 for (int b = 0; b < MT; ++b) acc[t][b] += red[(t * MT + b) * 64];
         }
     }
-    finish_unit<MT, NT, C::WM * C::WN>(acc, wk == 0, wm * C::WN + wn, lane, tid, splits, tile, unit, ws, locks, last_flag, y, M, N,
+    finish_unit<MT, NT, C::WM * C::WN, 64, C::FRAGS>(acc, wk == 0, wm * C::WN + wn, lane, tid, splits, tile, unit, ws, locks, last_flag, y, M, N,
                                  m0 + wm * 16 * MT, tile0 + wn * NT, tiles_n, act);
 }
 
