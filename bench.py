@@ -44,7 +44,8 @@ M = 16 the dequantize + torch.matmul comparator. Each shape rotates over enough 
 (>= 1 GB) that every call streams from HBM.
 
 `tune` times every compiled configuration of the chosen kernels per (shape, M) and prints the
-fastest (how layers/w4_tables.py was measured). `prof` is a fixed eager launch sequence for
+fastest (how layers/w4_tables.py was measured). `fit` fits the cost model of csrc/tw4_plan.hip to
+such records. `prof` is a fixed eager launch sequence for
 hardware-counter runs under rocprofv3, and summarizes their CSV files (see prof_main). `floor` times
 the plain-read ceiling (tw4_read_probe) at each projection's byte count (see read_floor).
 """
@@ -556,7 +557,8 @@ def tune_main(argv=None) -> int:
 
         python bench.py tune --model qwen3-8b --ms 1,4,8,16 --kinds gemv,mma [--out sweep.jsonl]
         python bench.py tune --model qwen3-8b --ms 24,32,64,256 --kinds gemm
-        python bench.py tune --model qwen3-8b --projs lm_head --ms 1,2,4,8 --kinds dense16,torch16
+        python bench.py tune --model qwen3-8b --projs lm_head --ms 1,2,4,8 --kinds dense16,gemm16,torch16
+        python bench.py tune --shapes 4096x6144,4096x24576 --ms 17,65,300 --kinds mma,gemm,tiled,dense --out sweep.jsonl
 
     For each projection shape and M, every compiled configuration of each kernel is timed the way the
     reference timed them (benchmarks/bench_gemv.py:35-56): one HIP graph replays `rounds` passes over
@@ -570,8 +572,10 @@ def tune_main(argv=None) -> int:
     ap = argparse.ArgumentParser(prog="bench.py tune", description=tune_main.__doc__.split("\n\n")[0])
     ap.add_argument("--model", default="qwen3-8b", choices=sorted(TUNE_MODELS))
     ap.add_argument("--projs", default="", help="comma list of projections (default: all)")
+    ap.add_argument("--shapes", default="", help="comma list of KxN, in place of a model's projections")
     ap.add_argument("--ms", default="1,4,8,16")
-    ap.add_argument("--kinds", default="gemv,mma", help="gemv, gemvm, gemvn, mma, mmak, mmap, gemm, dense")
+    ap.add_argument("--kinds", default="gemv,mma", help="gemv, gemvm, gemvn, mma, mmak, mmap, gemm, tiled, dense; lm_head: "
+                                                        "dense16, gemm16, torch16")
     ap.add_argument("--splits", default="0,1,2,4,8")
     ap.add_argument("--per-cu", default="1,2,3,4", help="workgroups per CU of the persistent mma (kind mmap)")
     ap.add_argument("--act", action="store_true", help="time the SwiGLU epilogue (gate_up only)")
@@ -621,11 +625,12 @@ def tune_main(argv=None) -> int:
         except RuntimeError:  # a configuration the host checks refuse for this shape
             pass
 
-    for proj, (k, n) in TUNE_MODELS[a.model].items():
-        if (a.projs and proj not in a.projs.split(",")) or (a.act and proj != "gate_up"):
+    shapes = {t: tuple(map(int, t.split("x"))) for t in a.shapes.split(",")} if a.shapes else TUNE_MODELS[a.model]
+    for proj, (k, n) in shapes.items():
+        if (a.projs and proj not in a.projs.split(",")) or (a.act and proj != "gate_up" and not a.shapes):
             continue
         act = int(a.act)
-        if (proj in DENSE) != any(kd in kinds for kd in ("dense16", "torch16")):
+        if (proj in DENSE) != any(kd in kinds for kd in ("dense16", "gemm16", "torch16")):
             continue
         if proj in DENSE:  # fp16 weights [N, K]: the kernel of layers/gemv16.py against F.linear
             from tandem_amd.layers import gemv16
@@ -639,6 +644,8 @@ def tune_main(argv=None) -> int:
                 if "dense16" in kinds:
                     for cfg in w4_hip.gemv_f16_configs():
                         attempt(res, ("dense16", *cfg), [lambda w=w, c=cfg: gemv16.gemv(x, w, *c) for w in wd], 3)
+                if "gemm16" in kinds and m <= gemv16.GEMM_MAX_ROWS:
+                    attempt(res, ("gemm16",), [lambda w=w: gemv16.gemm(x, w) for w in wd], 3)
                 if "torch16" in kinds:
                     attempt(res, ("torch16",), [lambda w=w: torch.nn.functional.linear(x, w) for w in wd], 3)
                 emit(proj, k, n, m, 0, copies, res, wbytes + 2 * m * k + 2 * m * n)
@@ -684,6 +691,13 @@ def tune_main(argv=None) -> int:
                             attempt(res, ("gemm", *cfg, sp),
                                     [lambda w=w, c=cfg, s=sp: ext.w4_gemm(x, *w, buf, locks, *c, s, act) for w in ws],
                                     5)
+            if "tiled" in kinds:
+                for cfg in w4_hip.gemm_tiled_configs():
+                    for sp in (int(v) for v in a.splits.split(",")):
+                        if sp <= k // 128:
+                            attempt(res, ("tiled", *cfg, sp),
+                                    [lambda w=w, c=cfg, s=sp: ext.w4_gemm_tiled(x, *w, buf, locks, *c, s, act) for w in ws],
+                                    5)
             if "dense" in kinds:  # HIP dequantize + torch.matmul, the unfused comparator
                 from tandem_amd.layers import awq
 
@@ -697,6 +711,107 @@ def tune_main(argv=None) -> int:
         torch.cuda.empty_cache()
     if out:
         out.close()
+    return 0
+
+
+# -------------------------------------------------------------------------------------- fit
+# What tw4_plan.hip predicts: the configurations it chooses among and the workgroups of each that share a CU
+FIT_OCC = {("tiled", 2, 2, 2, 1, 2, 4): 4, ("tiled", 2, 3, 2, 1, 2, 4): 4, ("tiled", 3, 2, 2, 1, 2, 4): 4,
+           ("tiled", 3, 3, 2, 1, 2, 4): 3, ("tiled", 4, 2, 2, 1, 2, 4): 3, ("tiled", 4, 3, 2, 1, 2, 4): 3,
+           ("tiled", 5, 2, 2, 1, 2, 4): 2, ("tiled", 5, 3, 2, 1, 2, 4): 2, ("tiled", 5, 4, 2, 1, 2, 4): 2,
+           ("tiled", 8, 2, 2, 1, 2, 4): 2, ("tiled", 8, 3, 2, 1, 2, 4): 1, ("tiled", 8, 4, 2, 1, 2, 4): 1,
+           ("tiled", 8, 4, 4, 1, 1, 3): 2, ("tiled", 8, 6, 2, 1, 2, 4): 1, ("tiled", 8, 6, 2, 2, 1, 3): 1,
+           ("gemm", 2, 1, 4, 2, 2): 4, ("gemm", 2, 2, 4, 2, 2): 2, ("gemm", 4, 2, 4, 2, 2): 2,
+           ("mma", 4, 1, 1): 2, ("mma", 4, 1, 2): 2, ("mma", 4, 1, 3): 2, ("mma", 4, 1, 6): 2}
+FIT_DENSE_ROWS = 1536
+
+
+def fit_terms(cfg: tuple, m: int, n: int, k: int, act: int, splits: int, cus: int = 256) -> list[float]:
+    """The terms tw4_gemm_plan multiplies a configuration's coefficients with, in the order of its rows."""
+    up = lambda a, b: -(-a // b)  # noqa: E731
+    if cfg[0] == "dense":
+        rounds = up(up(m, 256) * up(n, 256), cus)
+        return [1.0, n * k / 1e6, m * n * k / 1e9, rounds * k / 1e3, m * n / 1e6, act * m * n / 1e6]
+    occ, groups = FIT_OCC[cfg], k // 128
+    if cfg[0] == "mma":
+        bm, bn, steps = 64, 16 * cfg[3], up(groups, cfg[1])
+    elif cfg[0] == "tiled":
+        bm, bn, steps = 16 * cfg[1] * cfg[4], 16 * cfg[2] * cfg[3], 2 * up(groups, splits)
+    else:
+        bm, bn, steps = 16 * cfg[1], 16 * cfg[2] * cfg[3], up(up(groups, cfg[4]), splits)
+    tiles = up(m, bm) * up(n, bn)
+    units = up(tiles * splits, cus)
+    rounds, left = divmod(units, occ)
+    share = (left - 1) / (occ - 1) if left and occ > 1 else 0.0
+    full, alone = (rounds + share) * steps, (1.0 - share) * steps if left else 0.0
+    x_mb, act_mb = tiles * min(bm, m) * k * 2 / 1e6, act * m * n * 2 / 1e6
+    if cfg[0] == "mma":
+        mt = 2 if m <= 32 else 4
+        return [1.0, full, alone, full * mt, alone * mt, units - 1, mt, n * k / 2e6, x_mb, act_mb]
+    part, s = splits * bm * bn, float(splits > 1)
+    return [1.0, full, alone, units - 1, s, s * part / 1e4, n * k / 2e6, s * tiles * part * 4 / 1e6, x_mb,
+            up(m, bm) * n * k / 2e6, act_mb]
+
+
+def fit_main(argv=None) -> int:
+    """The coefficients of the M > 16 rule (csrc/tw4_plan.hip) from `tune` records, and how close the built library's
+    choices come to the fastest timed configuration:
+
+        python bench.py tune --shapes 4096x6144,... --ms 17,20,... --kinds mma,gemm,tiled,dense --splits 1,2,3,4,6,8,12,16 \\
+            --footprint-mb 500 --out sweep.jsonl            # and once more with --act for SwiGLU
+        python bench.py fit sweep.jsonl [--hold 8192x10240,...]
+
+    Non-negative least squares on relative errors, reweighted three times by 1 / (1 + (error / 15 %)^2), so that a few odd
+    sizes do not bend a row. --hold: shapes left out of the fit, reported on their own."""
+    import numpy as np
+    from scipy.optimize import nnls
+
+    from tandem_amd.layers import w4_plan
+
+    ap = argparse.ArgumentParser(prog="bench.py fit", description=fit_main.__doc__.split("\n\n")[0])
+    ap.add_argument("records", nargs="+")
+    ap.add_argument("--hold", default="")
+    a = ap.parse_args(argv)
+    hold = {tuple(map(int, t.split("x"))) for t in a.hold.split(",") if t}
+    points: dict[tuple, dict[tuple, float]] = {}
+    for path in a.records:
+        for line in open(path, encoding="utf-8"):
+            r = json.loads(line)
+            to = points.setdefault((r["m"], r["n"], r["k"], r["act"]), {})
+            for name, us in r["all"].items():
+                kind, *rest = name.split("/")
+                to[(kind, *map(int, rest))] = us
+    rows: dict[tuple, list] = {}
+    for (m, n, k, act), times in points.items():
+        if (k, n) in hold:
+            continue
+        for cfg, us in times.items():
+            c, sp = (cfg, 1) if cfg[0] in ("mma", "dense") else (cfg[:-1], cfg[-1])
+            if sp and (c in FIT_OCC or (c == ("dense",) and m >= FIT_DENSE_ROWS)):
+                rows.setdefault(c, []).append((fit_terms(c, m, n, k, act, sp), us))
+    for c in [*FIT_OCC, ("dense",)]:
+        if c not in rows:
+            continue
+        terms, us = (np.array(v, dtype=float) for v in zip(*rows[c]))
+        weight = 1 / us
+        x = nnls(terms * weight[:, None], us * weight)[0]
+        for _ in range(0 if c == ("dense",) else 3):
+            w = weight / (1 + ((terms @ x / us - 1) / 0.15) ** 2)
+            x = nnls(terms * w[:, None], us * w)[0]
+        err = terms @ x / us - 1
+        print(f"{'/'.join(map(str, c)):24s} {len(us):5d} calls, rms {np.sqrt((err ** 2).mean()):.3f}: "
+              f"{{{', '.join(f'{v:.4g}' for v in x)}}}")
+    for what, keep in (("fitted", lambda kn: kn not in hold), ("held out", lambda kn: kn in hold)):
+        over = []
+        for (m, n, k, act), times in points.items():
+            if keep((k, n)):
+                e = w4_plan.choose(m, n, k, bool(act))
+                e = ("dense",) if e is None else e if e[0] in ("mma", "tiled") else ("gemm", *e)
+                if e in times:
+                    over.append(times[e] / min(times.values()))
+        if over:
+            print(f"the built rule, {what}: {len(over)} sizes, {np.mean(over) - 1:.1%} over the fastest on average, 95 of 100 within "
+                  f"{np.quantile(over, 0.95) - 1:.1%}, {max(over) - 1:.0%} at worst")
     return 0
 
 
@@ -990,6 +1105,8 @@ def summarize_counters(paths: list[str], launches: int, kernel: str = "") -> dic
 if __name__ == "__main__":
     if len(sys.argv) > 1 and sys.argv[1] == "tune":
         sys.exit(tune_main(sys.argv[2:]))
+    if len(sys.argv) > 1 and sys.argv[1] == "fit":
+        sys.exit(fit_main(sys.argv[2:]))
     if len(sys.argv) > 1 and sys.argv[1] == "prof":
         sys.exit(prof_main(sys.argv[2:]))
     if len(sys.argv) > 1 and sys.argv[1] == "floor":

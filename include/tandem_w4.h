@@ -220,6 +220,16 @@ int tw4_gemm_tiled(const uint16_t* x, const int32_t* packed, const uint16_t* sca
 /* Compiled (mt, nt, warps_n, warps_m, warps_k, ring) configurations of tw4_gemm_tiled; returns how many. */
 int tw4_gemm_tiled_configs(int* out, int max_configs);
 
+/* The fastest kernel by size for y[M, N] = x[M, K] W^T, M > 16, on a device of `cus` CUs, where no measured table names one:
+ * writes its kind and arguments to out (room for 8) and returns how many it wrote, or a negative TW4_E code.
+ *   0                                                  dequantize + a dense product
+ *   1, warps_k, unroll, ntile                          tw4_mma
+ *   2, mt, nt, warps_n, warps_k, stages, splits        tw4_gemm
+ *   3, mt, nt, warps_n, warps_m, warps_k, ring, splits tw4_gemm_tiled
+ * Splits stay within TW4_AUTO_SPLIT_FLOATS and TW4_AUTO_SPLIT_COUNTERS. Host code, no device is touched. No reference
+ * counterpart (python/tandem/layers/awq.py:163-193 has fixed defaults). */
+int tw4_gemm_plan(int M, int N, int K, int act, int cus, int* out);
+
 /* tw4_gemm without a caller workspace, for callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc). No counterpart in the
  * reference. Same kernels, arguments (minus ws / locks / sizes), results and errors as tw4_gemm

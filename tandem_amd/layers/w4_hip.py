@@ -60,6 +60,7 @@ _SIGNATURES = {
     "tw4_capture_id": ([_P], ctypes.c_uint64),
     "tw4_gemm_tiled": ([_P, _P, _P, _P, _P, _P, _P, _I64, _I64, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _I, _P], _I),
     "tw4_gemm_tiled_configs": ([ctypes.POINTER(_I), _I], _I),
+    "tw4_gemm_plan": ([_I, _I, _I, _I, _I, ctypes.POINTER(_I)], _I),
     "tw4_gemm_last_grid": ([ctypes.POINTER(_I)] * 3, _I),
     "tw4_read_probe": ([_P, _I64, _I, _I, _I, ctypes.c_uint32, _P, _P], _I),
     "tw4_decode_configs": ([ctypes.POINTER(_I), _I], _I),

@@ -259,7 +259,7 @@ def test_tables_are_well_formed():
     assert awq.DEFAULT_KERNEL[0] in ("gemv", "mma") and len(awq.DEFAULT_KERNEL) == 4
     decode = set(w4_hip.decode_configs())
     mma = set(w4_hip.mma_configs())  # w4_mma also takes the row-tile-wide configs
-    gemm = set(w4_hip.gemm_configs())
+    gemm, tiled = set(w4_hip.gemm_configs()), set(w4_hip.gemm_tiled_configs())
     for table in awq.W4_KERNELS.values():
         for key, cfg in table.items():
             assert key[3:] in ((), ("silu",), ("norm",), ("silu", "norm"))
@@ -284,6 +284,7 @@ def test_tables_are_well_formed():
         assert m_maxes == sorted(m_maxes)
         for m_max, cfg in ladder:
             assert cfg is None or (len(cfg) == 6 and tuple(cfg[:5]) in gemm) or \
+                (cfg[0] == "tiled" and tuple(cfg[1:7]) in tiled and 0 <= cfg[7] <= 16) or \
                 (cfg[0] == "mma" and tuple(cfg[1:]) in mma and m_max <= 64 and cfg[2] * -(-m_max // 16) <= 4)
 
 

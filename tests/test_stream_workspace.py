@@ -88,12 +88,12 @@ def test_a_graph_runner_keeps_none():
         t.copy_(torch.randint(-2**31, 2**31 - 1, t.shape, device="cuda", dtype=torch.int32, generator=g))
     layer.scales.copy_((torch.rand(layer.scales.shape, device="cuda", generator=g) * 0.01).half())
     layer.finalize(torch.cuda.get_device_name())
-    assert layer.gemm_entry(24)[-1] != 1 and layer.gemm_entry(40)[-1] != 1
+    assert layer.gemm_entry(40)[-1] != 1 and layer.gemm_entry(48)[-1] != 1
     emb = torch.randn(100, k, device="cuda", generator=g).half()
     w4_hip._stream_workspaces.clear()
-    runner = decode_graph.DecodeGraphRunner(lambda ids: layer(emb[ids]), 40, torch.device("cuda", 0), logits=False)
+    runner = decode_graph.DecodeGraphRunner(lambda ids: layer(emb[ids]), 48, torch.device("cuda", 0), logits=False)
     assert not w4_hip._stream_workspaces
-    for b in (40, 24, 31, 3, 40):
+    for b in (48, 40, 33, 3, 47):
         ids = torch.randint(0, 100, (b,), generator=torch.Generator().manual_seed(b))
         bucket = runner.bucket(b)
         padded = torch.zeros(bucket, dtype=torch.long)
