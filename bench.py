@@ -29,7 +29,7 @@ value = whole-step algorithmic HBM bytes / time (GB/s), with the per-call byte c
                 max |ref| and cosine; parity_vs_dense holds the worst of them), and at M = 32 that
                 comparator's time
   full_stack    the whole decode step of the linears plus the fp16 lm_head (4096 x 151936, through
-                layers/gemv16.py's table: the HIP fp16 GEMV where it has an entry, else F.linear),
+                layers/gemv16.py: tw4_gemv_f16, tw4_gemm_f16 or F.linear, named by `lm_head`),
                 M in {1, 8, 32}: us per step and GB/s
   decode_step   tandem_amd.model's decode step replayed from the bucketed HIP graphs of
                 tandem_amd.decode_graph: norms, SwiGLU gate_up, lm_head and a ONE-TOKEN ATTENTION
@@ -510,7 +510,7 @@ def main(argv=None) -> int:
             b = a.layers * sum(call_bytes(mm, k, n) for _, k, n in QWEN3_8B) + 2 * hn * hk + 2 * mm * (hk + hn)
             full[f"m{mm}"] = {"us_per_step": round(us, 1), "GBps": round(b / us / 1e3, 1),
                               "pct_hbm_peak": round(b / us / 1e3 / HBM_PEAK_GBS * 100, 1), "step_bytes": b,
-                              "lm_head": "gemv16" if gemv16.entry(xd[4096], head, table) else "F.linear"}
+                              "lm_head": gemv16.route(xd[4096], head, table)}
         del head
         torch.cuda.synchronize()
 

@@ -150,6 +150,7 @@ def gemm(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 # K = 4160 0.62-0.92; the rows of x, read from L2 for every 64 of w, pass it at M > 24 and K = 12288 (49152 columns 1.05).
 GEMM_MIN_BYTES = 128 << 20
 GEMM_MAX_ROWS = 32
+GEMM = ("gemm",)  # the choice of tw4_gemm_f16
 
 
 def streams(m: int, n: int, k: int) -> bool:
@@ -176,19 +177,35 @@ def linear(x: torch.Tensor, w: torch.Tensor, table: dict[tuple[int, int, int], C
     tw4_gemm_f16 where streaming w bounds it (the logits head at every other batch up to 32 and every other size; up to
     M = 4, whose x the vector form keeps in LDS whole, tw4_gemv_f16 where it takes K: 184 us against 197 on the Qwen3-8B
     head at M = 1), through F.linear (hipBLASLt) otherwise (python/tandem/layers/triton_gemv.py:285-297)."""
+    cfg = _choice(x, w, table, eager)
+    if cfg is None:
+        return F.linear(x, w)
+    return gemm(x, w) if cfg == GEMM else gemv(x, w, *cfg)
+
+
+def _choice(x: torch.Tensor, w: torch.Tensor, table: dict[tuple[int, int, int], Config], eager: bool) -> tuple | None:
+    """What ``linear`` runs: a configuration of gemv, GEMM, or None for F.linear."""
     cfg = entry(x, w, table, eager)
-    if cfg is not None and not (w4_hip.plain(x) and w4_hip.plain(w)):
-        return F.linear(x, w)  # a gradient or a transform follows the call
+    if cfg is not None:  # unless a gradient or a transform follows the call
+        return cfg if w4_hip.plain(x) and w4_hip.plain(w) else None
+    if not (eager and table and _streams(x, w)):
+        return None
     # F.linear's own result where autocast, a mode or a compiler would change it; a shape the table names stays a kernel up to
     # its last bucket
-    named = x.dim() == 2 and x.shape[0] <= BUCKETS[-1] and (*w.shape, 4) in table
-    if cfg is None and eager and table and _streams(x, w) and (named or not w4_hip.intercepted()):
-        if x.shape[0] > 4 or x.shape[1] not in KS:
-            return gemm(x, w)
-        # rows per wavefront: 32 for the long rows of K = 4096 (20480 columns 0.49 against 0.59 of F.linear's time at M = 1),
-        # 16 for shorter ones and few columns, where they leave wavefronts short (1024 x 102400 at M = 4 1.06 against 0.92)
-        cfg = (2, 32) if w.shape[1] > 2048 and w.shape[0] >= 20480 else (2, 16)
-    return F.linear(x, w) if cfg is None else gemv(x, w, *cfg)
+    m, (n, k) = x.shape[0], w.shape
+    if w4_hip.intercepted() and not (m <= BUCKETS[-1] and (n, k, 4) in table):
+        return None
+    if m > 4 or k not in KS:
+        return GEMM
+    # rows per wavefront: 32 for the long rows of K = 4096 (20480 columns 0.49 against 0.59 of F.linear's time at M = 1),
+    # 16 for shorter ones and few columns, where they leave wavefronts short (1024 x 102400 at M = 4 1.06 against 0.92)
+    return (2, 32) if k > 2048 and n >= 20480 else (2, 16)
+
+
+def route(x: torch.Tensor, w: torch.Tensor, table: dict[tuple[int, int, int], Config], eager: bool = True) -> str:
+    """The kernel ``linear`` runs for these tensors, by the same lookups."""
+    cfg = _choice(x, w, table, eager)
+    return "F.linear" if cfg is None else "tw4_gemm_f16" if cfg == GEMM else f"tw4_gemv_f16{cfg}"
 
 
 class TabledLinear(nn.Linear):

@@ -67,12 +67,12 @@ def test_linear_takes_it_where_streaming_w_bounds(monkeypatch):
     for m, want in ((1, "gemv"), (4, "gemv"), (5, "gemm"), (32, "gemm")):
         calls.clear()
         _check(gemv16.linear(x[:m], w, table), x[:m], w)
-        assert calls == [want], m
+        assert calls == [want] and gemv16.route(x[:m], w, table).startswith(f"tw4_{want}_f16"), m
     calls.clear()
     short, wide = w[:4096], torch.cat([x, x])
     strided = torch.cat([x, x], dim=1)[:, :2048]
     for xx, ww, t in ((x, short, table), (wide, w, table), (strided, w, table), (x, w, {}), (x[:0], w, table)):
-        assert torch.equal(gemv16.linear(xx, ww, t), F.linear(xx, ww))
+        assert torch.equal(gemv16.linear(xx, ww, t), F.linear(xx, ww)) and gemv16.route(xx, ww, t) == "F.linear"
     xg = x.clone().requires_grad_()
     gemv16.linear(xg, w, table).sum().backward()
     assert xg.grad is not None and not calls
