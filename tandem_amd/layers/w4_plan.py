@@ -33,35 +33,41 @@ DECODE_MAX_K = 17408  # the largest K the rule was timed at
 
 def decode(m: int, n: int, k: int, cus: int = 256) -> tuple | None:
     """The decode kernel for 1 <= m <= 16 rows of a shape without table entries, None where the fixed
-    choice mma (4, 2, 1) is as good. From 12 shapes (K 1024 .. 16384, N 1032 .. 24000) x M = 1, 2, 4, 8, 16 x every
-    compiled matrix-core configuration on MI355X, 256 CUs, weights streamed from HBM; up to 2.2 times faster than the fixed
-    choice (one of the 60 points is slower, by 1 %).
-    us, fixed -> this choice:
+    choice mma (4, 2, 1) is as good. From 28 shapes (K 768 .. 17408, N 1032 .. 24000) x 12 M x 11 matrix-core configurations on
+    MI355X, 256 CUs, weights streamed from HBM (profiles/decode_rule_sweep.jsonl); at most 1.4 % slower than
+    the fixed choice anywhere, 0.91 of its time on average. Against it:
 
     Row tiles for two and more workgroups per CU (tiles > 2 CUs): reading x again for every 16 rows is what costs, so
-      several row tiles share a workgroup from M = 5 on: six from four tiles per CU (8192 x 20000 at M = 16 42.9 -> 22.6),
-      three below, where six leave CUs without a workgroup (4096 x 9000 14.3 -> 8.7); a short K (to 2048) is launch and
-      x staging instead and keeps one tile, 8 wavefronts, up to M = 12. M = 3, 4: two tiles (8192 x 20000 at M = 4
-      22.3 -> 19.3), three from K 4096 on between (13056 x 10240 22.9 -> 18.5).
-    One to two tiles per CU: two tiles per workgroup fill each CU once (8192 x 5000 at M = 16 18.0 -> 11.3).
-    At most one tile per CU: wavefronts, not x, are short: 16 of them while x fits LDS beside (m k <= 2^16; 16384 x 1536 at M = 4
-      10.4 -> 8.1), 8 for a short K.
+      several row tiles share a workgroup: with a long K from M = 5 on six from four tiles per CU (8192 x 20000 at M = 16
+      43.2 -> 21.3 us), three below, where six leave CUs without a workgroup (4096 x 9000 14.4 -> 8.7), two at M = 3, 4. A short K
+      (to 2048) is launch and x staging instead: 8 wavefronts up to M = 4 (1536 x 8960 at M = 3 4.73 -> 4.07) where the
+      workgroups are few, two tiles up to M = 8 (1792 x 12800 at M = 5 5.63 -> 5.41), three from M = 9 on (2048 x 10240 at M = 16
+      7.51 -> 5.85).
+    One to two tiles per CU: two tiles per workgroup fill each CU once (17408 x 5120 at M = 16 36.1 -> 22.4).
+    At most one tile per CU: wavefronts, not x, are short: 8 of them, for a long K while x fits LDS beside (m k <= 2^16; 17408 x 1536
+      at M = 2 11.0 -> 9.2).
 
-    Timed and left out: the vector-ALU GEMV at M = 1 (4096 x 9000 6.3 -> 5.4). It takes the 1024 of its magic halves off a sum
-    with x in it, so an infinite x gives NaN where the matrix cores give infinities; an eager call is bound by the host there."""
+    Timed and left out: 16 wavefronts at most one tile per CU (5120 x 3000 at M = 12 6.2 -> 7.4) and 8 of them for a short K at M = 5 .. 8
+    (2048 x 20000 at M = 5 7.0 -> 9.1), which an earlier form of the rule took from twelve shapes; and the vector-ALU GEMV at M = 1
+    (4096 x 9000 6.3 -> 5.4): it takes the 1024 of its magic halves off a sum with x in it, so an infinite x gives NaN where the
+    matrix cores give infinities."""
     if k > DECODE_MAX_K:
         return None
     tiles = _cdiv(n, 16)
     if tiles <= cus:
-        if k <= 2304:
-            return ("mma", 8, 1, 1)
-        return ("mma", 16, 2, 1) if m * k <= 1 << 16 else None
+        if k <= 1536:
+            return ("mma", 8, 1, 1) if m <= 8 else None
+        return ("mma", 8, 2, 1) if k > 2304 and m * k <= 1 << 16 else None
     if tiles <= 2 * cus:
-        if m < 4:
+        if m < 4 or (m == 4 and k < 2048):
             return None
         return ("mma", 8, 1, 2) if m <= 8 else ("mma", 4, 2, 2)
     if k <= 2048:
-        return ("mma", 8, 1, 1) if m <= 12 else ("mma", 4, 1, 3)
+        if m <= 4:
+            return ("mma", 8, 1, 1) if tiles < 4 * cus else None
+        if m <= 8:
+            return ("mma", 4, 1, 2) if k < 2048 else None
+        return ("mma", 4, 1, 3)
     if m < 3:
         return None
     if tiles >= 4 * cus:

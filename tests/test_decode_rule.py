@@ -27,6 +27,17 @@ def test_every_choice_is_compiled():
             assert e is None or (e[0] == "mma" and e[1:] in mma and k <= 17408), (m, n, k, e)
 
 
+def test_eight_and_sixteen_wavefronts_only_where_they_pay():
+    """Sizes where they take 1.1 to 1.4 of the fixed choice's time: many row tiles with a short K, and x past what leaves room
+    beside it."""
+    for m, n, k in ((1, 20000, 768), (10, 20000, 768), (9, 17000, 1024), (5, 20000, 2048), (6, 8960, 1536), (5, 12800, 1792),
+                    (12, 10240, 2048), (12, 3000, 5120), (3, 3000, 5120), (12, 3000, 2304), (4, 4864, 896), (10, 4096, 1024)):
+        e = w4_plan.decode(m, n, k)
+        assert e is None or e[1] == 4 or e == ("mma", 8, 2, 1), (m, n, k, e)
+    assert w4_plan.decode(3, 8960, 1536) == w4_plan.decode(8, 1032, 1152) == ("mma", 8, 1, 1)
+    assert w4_plan.decode(2, 1536, 17408) == ("mma", 8, 2, 1)
+
+
 def test_layers_without_a_table_keep_the_default():
     layer = awq.W4Linear(4096, 9000, 128)
     assert layer.decode_entry(16) == layer.norm_entry(1) == awq.DEFAULT_KERNEL
