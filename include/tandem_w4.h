@@ -82,6 +82,11 @@ int tw4_repack_awq(const int32_t* qweight, const int32_t* qzeros, const uint16_t
 int tw4_dequant(const int32_t* packed, const uint16_t* scales, const uint16_t* zeros,
                 uint16_t* out, int N, int K, int deinterleave, void* stream);
 
+/* tw4_dequant for a matrix that is read right after, by a dense product: the same values, stored so that a matrix the
+ * 256 MB cache in front of HBM holds is read from there (tw4_dequant's own stores pass it by). */
+int tw4_dequant_near(const int32_t* packed, const uint16_t* scales, const uint16_t* zeros,
+                     uint16_t* out, int N, int K, int deinterleave, void* stream);
+
 /* Decode GEMV on the vector ALUs, 1 <= M <= 4: y fp16 [M, N]. x fp16 [M, K] contiguous and
  * 16-byte aligned. Config: warps_k wavefronts split K into contiguous group ranges inside a
  * workgroup, unroll quant groups per chunk (one chunk in flight ahead of the math), ntile row

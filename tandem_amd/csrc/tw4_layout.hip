@@ -100,11 +100,15 @@ __global__ void __launch_bounds__(256) repack_kernel(const uint32_t* __restrict_
 
 // Dense weights: a workgroup takes 16 rows (one tile) x 512 k (four groups; fewer at the end of a row), a wavefront one
 // group of 128 k: each lane dequantizes its 16 bytes (32 weights of one row) and parks them in LDS, and the workgroup
-// writes the 16 rows' 1 KB pieces with whole lines per instruction (a wavefront store is one row's 1 KB), non-temporal:
-// the matrix is far larger than the caches and its reader comes after it whole. LDS rows are 65 chunks of 16 bytes, so
-// the 16 rows of a column of chunks sit in different banks.
-// Bound by memory. Against four 16-byte stores per lane 64 bytes apart: Qwen3-8B down (12288 x 4096) 36.7 -> 22.4 us
-// (5.8 TB/s), gate_up (4096 x 24576) 73 -> 41.
+// writes the 16 rows' 1 KB pieces with whole lines per instruction (a wavefront store is one row's 1 KB). LDS rows are 65
+// chunks of 16 bytes, so the 16 rows of a column of chunks sit in different banks.
+// Bound by memory. Against four 16-byte stores per lane 64 bytes apart: Qwen3-8B down (12288 x 4096) 36.5 -> 22.3 us
+// (5.9 TB/s), gate_up (4096 x 24576) 74 -> 41.
+// STREAM: non-temporal stores, for a matrix that is kept or exceeds the 256 MB cache in front of HBM. Plain ones leave a smaller
+// one there for the product that reads it next: dequantize + product of 5120 x 7168 at M = 4096 259 -> 234 us (244 with the
+// strided stores), 17408 x 5120 at M = 100 183 -> 144; the dequantization alone takes up to 15 % longer (4096 x 6144 11.2 -> 12.9).
+// 5120 x 34816 (356 MB) is faster non-temporal all the way: 1303 against 1320 at M = 4096.
+template <bool STREAM>
 __global__ void __launch_bounds__(256) dequant_kernel(const u4* __restrict__ packed, const h1* __restrict__ scales,
                                                       const h1* __restrict__ zeros, u4* __restrict__ out, int N, int K,
                                                       int pieces, int deinterleave) {
@@ -132,7 +136,11 @@ __global__ void __launch_bounds__(256) dequant_kernel(const u4* __restrict__ pac
             const int rr = 4 * wave + i, row = 16 * t + rr;
             if (rr >= rows) break;
             const int dst = deinterleave ? interleaved_source_row(row, N) : row;
-            __builtin_nontemporal_store(tile[65 * rr + lane], out + static_cast<int64_t>(dst) * (K >> 3) + 16 * g0 + lane);
+            u4* o = out + static_cast<int64_t>(dst) * (K >> 3) + 16 * g0 + lane;
+            if constexpr (STREAM)
+                __builtin_nontemporal_store(tile[65 * rr + lane], o);
+            else
+                *o = tile[65 * rr + lane];
         }
     }
 }
@@ -164,7 +172,8 @@ extern "C" int tw4_repack_awq(const int32_t* qweight, const int32_t* qzeros, con
     return TW4_OK;
 }
 
-extern "C" int tw4_dequant(const int32_t* packed, const uint16_t* scales, const uint16_t* zeros, uint16_t* out,
+template <bool STREAM>
+static int dequant_launch(const int32_t* packed, const uint16_t* scales, const uint16_t* zeros, uint16_t* out,
                            int N, int K, int deinterleave, void* stream) {
     TW4_REQUIRE(K > 0 && K % 128 == 0, TW4_EINVAL, "dequant: K %% 128 == 0 (K = %d)", K);
     TW4_REQUIRE(N > 0 && N % 8 == 0, TW4_EINVAL, "dequant: N %% 8 == 0 (N = %d)", N);
@@ -175,9 +184,19 @@ extern "C" int tw4_dequant(const int32_t* packed, const uint16_t* scales, const 
     const int pieces = ((K >> 7) + 3) / 4;
     const int64_t blocks = static_cast<int64_t>((N + 15) >> 4) * pieces;
     TW4_REQUIRE(blocks < (1LL << 31), TW4_EINVAL, "dequant: grid too large");
-    dequant_kernel<<<static_cast<unsigned>(blocks), 256, 0, static_cast<hipStream_t>(stream)>>>(
+    dequant_kernel<STREAM><<<static_cast<unsigned>(blocks), 256, 0, static_cast<hipStream_t>(stream)>>>(
         reinterpret_cast<const u4*>(packed), reinterpret_cast<const h1*>(scales), reinterpret_cast<const h1*>(zeros),
         reinterpret_cast<u4*>(out), N, K, pieces, deinterleave);
     TW4_LAUNCH_CHECK("dequant: launch");
     return TW4_OK;
+}
+
+extern "C" int tw4_dequant(const int32_t* packed, const uint16_t* scales, const uint16_t* zeros, uint16_t* out, int N, int K,
+                           int deinterleave, void* stream) {
+    return dequant_launch<true>(packed, scales, zeros, out, N, K, deinterleave, stream);
+}
+
+extern "C" int tw4_dequant_near(const int32_t* packed, const uint16_t* scales, const uint16_t* zeros, uint16_t* out, int N,
+                                int K, int deinterleave, void* stream) {
+    return dequant_launch<false>(packed, scales, zeros, out, N, K, deinterleave, stream);
 }

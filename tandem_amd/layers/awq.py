@@ -287,8 +287,8 @@ class W4Linear(nn.Module):
         activation as the unfused path (python/tandem/layers/awq.py:282-286)."""
         if not x.is_cuda:
             raise RuntimeError("W4Linear: x must be on the GPU (there is no CPU path)")
-        w = w4_dequant(self.packed, self.scales, self.zeros, self.group, x.dtype, deinterleave=self.silu_mul)
-        y = F.linear(x, w)
+        w = w4_hip.dequant(self.packed, self.scales, self.zeros, deinterleave=self.silu_mul, near=True)
+        y = F.linear(x, w if x.dtype == torch.float16 else w.to(x.dtype))
         return silu_and_mul(y) if self.silu_mul else y
 
     def _gemm(self, ext, x: torch.Tensor, cfg) -> torch.Tensor:

@@ -49,6 +49,7 @@ _SIGNATURES = {
     "tw4_init": ([_I], _I),
     "tw4_repack_awq": ([_P, _P, _P, _P, _P, _P, _I, _I, _I, _P], _I),
     "tw4_dequant": ([_P, _P, _P, _P, _I, _I, _I, _P], _I),
+    "tw4_dequant_near": ([_P, _P, _P, _P, _I, _I, _I, _P], _I),
     "tw4_gemv": ([_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _P], _I),
     "tw4_gemv_act": ([_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P], _I),
     "tw4_gemv_mfma": ([_P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _I, _I, _P], _I),
@@ -402,8 +403,13 @@ def repack(qweight: torch.Tensor, qzeros: torch.Tensor, scales: torch.Tensor,
     return packed, s_out, z_out
 
 
-def dequant(packed: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor, deinterleave: bool = False) -> torch.Tensor:
-    """Tile layout -> dense fp16 [N, K] (bit-exact fp16_rne((q - z) s)) by the tw4_dequant kernel."""
+NEAR_BYTES = 256 << 20  # what the cache in front of HBM holds
+
+
+def dequant(packed: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor, deinterleave: bool = False,
+            near: bool = False) -> torch.Tensor:
+    """Tile layout -> dense fp16 [N, K] (bit-exact fp16_rne((q - z) s)) by the tw4_dequant kernel. near: it is read right
+    after, so its stores go through the cache if it fits there (tw4_dequant_near)."""
     if not (packed.is_cuda and scales.is_cuda and zeros.is_cuda):
         raise RuntimeError("w4_dequant: tensors must be on the GPU")
     n, g = scales.shape
@@ -415,8 +421,8 @@ def dequant(packed: torch.Tensor, scales: torch.Tensor, zeros: torch.Tensor, dei
                            f"scales / zeros [N, K/128] (got {tuple(packed.shape)}, {tuple(scales.shape)})")
     out = torch.empty((n, k), dtype=torch.float16, device=packed.device)
     with on_device(packed.get_device()):
-        check(library().tw4_dequant(_ptr(packed), _ptr(scales), _ptr(zeros), _ptr(out), n, k,
-                                    int(bool(deinterleave)), _stream(packed)))
+        call = library().tw4_dequant_near if near and 2 * n * k <= NEAR_BYTES else library().tw4_dequant
+        check(call(_ptr(packed), _ptr(scales), _ptr(zeros), _ptr(out), n, k, int(bool(deinterleave)), _stream(packed)))
     return out
 
 

@@ -47,5 +47,6 @@ def test_repack_and_dequant_tile_edges(k, n, shift):
         assert (store.cpu()[:int(shift)] == -1).all() and (store.cpu()[words + int(shift):] == -1).all()
         assert torch.equal(s_out.cpu(), awq.tile_major_params(order(s)))
         assert torch.equal(z_out.cpu(), awq.tile_major_params(order(z)))
-        w = awq.w4_dequant(packed.clone().view(-1, k // 8), s_out, z_out, deinterleave=interleave)
-        assert np.array_equal(w.cpu().numpy().view(np.uint16), o.dequant(qweight, qzeros, scales).view(np.uint16))
+        for near in (False, True):
+            w = w4_hip.dequant(packed.clone().view(-1, k // 8), s_out, z_out, deinterleave=interleave, near=near)
+            assert np.array_equal(w.cpu().numpy().view(np.uint16), o.dequant(qweight, qzeros, scales).view(np.uint16))
