@@ -1,4 +1,4 @@
-"""The norm kernels over every compiled width and both forms (short and tall batches): a row's result is the same bits
+"""The norm kernels over every compiled width and every form (short and tall batches, four rows per workgroup): a row's result is the same bits
 whatever the batch, and within rounding of 64 bits (fp32 arithmetic: K 2^-23 relative for the sum of squares, a few units of
 2^-24 behind it, and half a unit in the last place of fp16, 2^-11; the residual is x + r rounded once)."""
 
@@ -21,7 +21,7 @@ def test_rows_do_not_depend_on_the_batch(k):
     w = (0.5 + torch.rand(k, device="cuda", generator=g)).half()
     want_y = norm.rms_norm(x0, w, EPS)
     want_x, want_r = norm.fused_add_rms_norm(x0.clone(), r0.clone(), w, EPS)
-    for m in (1, 3, 1023, 1024):
+    for m in (1, 3, 639, 640, 641, 642, 643, 1023, 1024):
         x, r = norm.fused_add_rms_norm(x0[-m:].clone(), r0[-m:].clone(), w, EPS)
         assert torch.equal(x, want_x[-m:]) and torch.equal(r, want_r[-m:])
         assert torch.equal(norm.rms_norm(x0[-m:].clone(), w, EPS), want_y[-m:])
