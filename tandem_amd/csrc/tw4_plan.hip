@@ -11,7 +11,7 @@
 // The coefficients are microseconds on MI355X (256 CUs), fitted with `python bench.py fit` (non-negative least squares on relative
 // errors) to 34,000 timed calls, weights streamed from HBM: 28 (K, N) from 1024 x 4096 to 5120 x 34816, N = 1032 and 7288
 // among them, x 35 M from 17 to 4096 (profiles/gemm_rule_sweep.jsonl). The choice is 1.2 % slower than the fastest timed
-// candidate on average, within 6 % at 95 of 100 sizes, 20 % at worst (a library product at M = 4096); 1.4, 8 and 22 % over seven shapes
+// candidate on average, within 6 % at 95 of 100 sizes, 16 % at worst; 1.4, 8 and 26 % (a library product at M = 3500) over seven shapes
 // left out of the fit. Against the fixed ladder these sizes had before any rule (8 wavefronts of the decode kernel up to M = 64, the
 // x-ring GEMM to 1024, dequantize + hipBLASLt above) it takes 0.72 of the time on average: Qwen3-14B gate_up at M = 40 132 us
 // against 40, Qwen3-8B-sized qkv (K 4096, N 6144) at M = 512 43 against 32.
@@ -64,7 +64,7 @@ constexpr PlanTiled kPlanTiled[] = {
     {8, 2, 2, 1, 2, 4, 2, {5.049, 0.4184, 0.2512, 1.612, 0, 0.8086, 0.0276, 0.2331, 0.008498, 0.03748, 0.4059}},  // 128 x 64
     {8, 3, 2, 1, 2, 4, 1, {6.235, 0.3184, 0, 5.066, 0, 0.3184, 0.04632, 0.256, 0.01242, 0.007974, 0.5946}},  // 128 x 96
     {8, 4, 2, 1, 2, 4, 1, {6.997, 0.3431, 0, 5.842, 0, 0.3484, 0.01823, 0.2542, 0.006154, 0.1048, 0.5239}},  // 128 x 128
-    {8, 4, 4, 1, 1, 3, 2, {7.752, 0.8929, 0.5034, 3.641, 0, 1.069, 0.03307, 0.1594, 0.004291, 0.1579, 0.1466}},  // 128 x 256
+    {8, 4, 4, 1, 1, 3, 2, {7.718, 0.8805, 0.4976, 3.692, 0, 0.4335, 0.04006, 0.2131, 0, 0.1692, 0.1435}},  // 128 x 256
     {8, 6, 2, 1, 2, 4, 1, {8.902, 0.4914, 0, 7.638, 0, 1.137, 0.05522, 0.2284, 0.0397, 0.006301, 0.5254}},  // 128 x 192
     {8, 6, 2, 2, 1, 3, 1, {9.728, 0.7085, 0, 10.48, 0, 0, 0.04363, 0.5105, 0.02484, 0.2178, 0.09126}},  // 256 x 192
 };
@@ -81,8 +81,10 @@ constexpr PlanMma kPlanMma[] = {
 };
 // dequantize + hipBLASLt, from M = 1536 on (below, a fused kernel was the fastest at every timed size): launches, per 10^6
 // weights (the dequantized matrix out and in), per 10^9 products, per round of 256 x 256 tiles and 10^3 k (its last round nearly
-// empty costs a whole one), per 10^6 results, and those of the separate SwiGLU
-constexpr double kPlanDense[6] = {10.12, 0.7475, 1.114, 3.094, 0.2807, 1.277};
+// empty costs a whole one), per 10^6 results, and those of the separate SwiGLU. At ragged M the library's time varies most (24576 x
+// 4096 at M = 3000 618 us, as at 4096, against 509 fused): there it has to be that much faster.
+constexpr double kPlanRagged = 1.03;
+constexpr double kPlanDense[6] = {10.4, 0.6708, 1.142, 2.327, 0.2666, 1.306};
 constexpr int kPlanDenseRows = 1536;
 constexpr int kPlanRingRows = 256;
 constexpr int kPlanSplits[] = {1, 2, 3, 4, 6, 8, 12, 16};
@@ -136,8 +138,9 @@ extern "C" int tw4_gemm_plan(int M, int N, int K, int act, int cus, int* out) {
     if (M >= kPlanDenseRows) {
         const double* d = kPlanDense;
         const double rounds = static_cast<double>(cdiv(cdiv(M, 256) * cdiv(N, 256), cus));
-        offer(d[0] + (d[1] * n * k / 1e6 + d[2] * m * n * k / 1e9 + d[4] * m * n / 1e6 + (act ? d[5] * m * n / 1e6 : 0.0)) * chip +
-                  d[3] * rounds * k / 1e3, {0});
+        const double t = d[0] + d[3] * rounds * k / 1e3 +
+                         (d[1] * n * k / 1e6 + d[2] * m * n * k / 1e9 + d[4] * m * n / 1e6 + (act ? d[5] * m * n / 1e6 : 0.0)) * chip;
+        offer(M % 256 ? kPlanRagged * t : t, {0});
     }
     if (static_cast<int64_t>(M) * K < (1LL << 31) && ((N + 15LL) & ~15LL) * K < (1LL << 33))  // tw4_gemm_tiled's limits
         for (const PlanTiled& p : kPlanTiled) {

@@ -66,7 +66,7 @@ def _cheapest(m: int, n: int, k: int, act: int, cus: int) -> dict[tuple | None, 
     if m >= bench.FIT_DENSE_ROWS:
         t = bench.fit_terms(("dense",), m, n, k, act, 1, cus)
         t[1:] = [v * scale if i != 2 else v for i, v in enumerate(t[1:])]
-        costs[None] = sum(a * b for a, b in zip(ROWS["dense",], t))
+        costs[None] = sum(a * b for a, b in zip(ROWS["dense",], t)) * (1.03 if m % 256 else 1.0)
     return costs
 
 
