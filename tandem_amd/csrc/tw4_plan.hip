@@ -11,7 +11,7 @@
 // The coefficients are microseconds on MI355X (256 CUs), fitted with `python bench.py fit` (non-negative least squares on relative
 // errors) to 34,000 timed calls, weights streamed from HBM: 28 (K, N) from 1024 x 4096 to 5120 x 34816, N = 1032 and 7288
 // among them, x 35 M from 17 to 4096 (profiles/gemm_rule_sweep.jsonl). The choice is 1.2 % slower than the fastest timed
-// candidate on average, within 6 % at 95 of 100 sizes, 16 % at worst; 1.4, 8 and 26 % (a library product at M = 3500) over seven shapes
+// candidate on average, within 6 % at 95 of 100 sizes, 16 % at worst; 1.5, 8 and 26 % (a library product at M = 3500) over seven shapes
 // left out of the fit. Against the fixed ladder these sizes had before any rule (8 wavefronts of the decode kernel up to M = 64, the
 // x-ring GEMM to 1024, dequantize + hipBLASLt above) it takes 0.72 of the time on average: Qwen3-14B gate_up at M = 40 132 us
 // against 40, Qwen3-8B-sized qkv (K 4096, N 6144) at M = 512 43 against 32.

@@ -243,6 +243,10 @@ class W4Linear(nn.Module):
     A SwiGLU MLP's gate_up calls ``enable_silu_mul`` before ``finalize``: the repack then interleaves
     gate and up rows by 8 and every kernel's epilogue returns silu(gate) * up, [M, out_features / 2]."""
 
+    # finalize's; class attributes, so that a layer pickled without them still runs (as it was: no rule up to M = 16)
+    cus = 256  # of the layer's GPU, for the rules
+    decode_rule = False  # w4_plan.decode for M <= 16 without an entry: on the GPUs that have a table
+
     def __init__(self, in_features: int, out_features: int, group: int) -> None:
         super().__init__()
         if group != 128 or in_features % group or out_features % 8:
@@ -256,8 +260,6 @@ class W4Linear(nn.Module):
         self.register_buffer("scales", torch.empty(in_features // group, out_features, dtype=torch.float16))
         self.kernels: dict[tuple, W4Kernel] = {}
         self.gemm_kernels: dict[tuple, tuple[tuple[int, W4Gemm | None], ...]] = {}
-        self.cus = 256  # of the layer's GPU, for the rules (finalize)
-        self.decode_rule = False  # w4_plan.decode for M <= 16 without an entry: on the GPUs that have a table
 
     def enable_silu_mul(self) -> bool:
         if not self.awq_layout or self.out_features % 16:

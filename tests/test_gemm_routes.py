@@ -68,6 +68,12 @@ def test_ladders_survive_a_copy_of_the_layer():
         assert all(a.fused_rows == b.fused_rows for a, b in zip(other.gemm_kernels.values(), GFX950_GEMM.values()))
 
 
+def test_a_layer_pickled_before_the_rules_runs():
+    layer = _layer(table={(6144, 4096): FIXED})
+    assert "cus" not in vars(layer) and "decode_rule" not in vars(layer)  # what such a pickle holds
+    assert layer.decode_entry(3) == awq.DEFAULT_KERNEL and layer.gemm_entry(300) == FIXED[1][1]
+
+
 @contextlib.contextmanager
 def _autocast(dtype):
     """torch.autocast("cuda", dtype) without the check for a GPU."""
