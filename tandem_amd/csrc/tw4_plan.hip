@@ -79,7 +79,7 @@ constexpr PlanMma kPlanMma[] = {
     {4, 1, 3, 64, 2.59, 0.3685, 0.1419, 0.4001, 0.3175, 0.5103, 0.1105, 0, 0.06497, 0.6496},
     {4, 1, 6, 64, 3.442, 0.7838, 0.3092, 0.7079, 0.3663, 0, 0.579, 0, 0.06583, 1.868},
 };
-// dequantize + hipBLASLt, from M = 1536 on (below, a fused kernel was the fastest at every timed size): launches, per 10^6
+// dequantize + hipBLASLt, from M = 1536 on (below, a fused kernel was the fastest at all but one of the timed sizes): launches, per 10^6
 // weights (the dequantized matrix out and in), per 10^9 products, per round of 256 x 256 tiles and 10^3 k (its last round nearly
 // empty costs a whole one), per 10^6 results, and those of the separate SwiGLU. At ragged M the library's time varies most (24576 x
 // 4096 at M = 3000 618 us, as at 4096, against 509 fused): there it has to be that much faster.

@@ -82,23 +82,23 @@ def test_qwen3_1_7b_tables(proj, silu):
 
 @pytest.mark.parametrize("proj,silu", [("qkv", False), ("o", False), ("gate_up", True), ("down", False)])
 def test_qwen3_8b_prefill_sizes(proj, silu):
-    """Qwen3-8B at M = 1024 and 4096 through the table (the fused GEMM, or dequantize + hipBLASLt
-    where the table says so) and a forced fused-GEMM configuration at M = 4096, on 512 sampled
+    """Qwen3-8B at M = 1024 and 4096 through the layer's choice (the tiled GEMM, or dequantize + hipBLASLt
+    where the rule says so) and a forced fused-GEMM configuration at M = 4096, on 512 sampled
     output features against the oracle's float64 product."""
     k, n = QWEN3_8B[proj]
     layer, t = awq_layer(k, n, seed=180 + len(proj), silu=silu)
     n_out = n // 2 if silu else n
     rng = np.random.default_rng(181)
     feats = np.sort(rng.choice(n_out, size=512, replace=False))
-    key = (n, k) + (("silu",) if silu else ())
-    table = layer.gemm_kernels.get(key, awq.DEFAULT_GEMM)
     buf, locks = w4_hip.workspace(DEV)
     ext = w4_hip.load()
     for m in (1024, 4096):
         x = rng.standard_normal((m, k)).astype(np.float16)
         xg = gpu(x)
         ref = sampled_reference(x, t, feats, n, silu)
-        runs = [("table", awq.pick_gemm(table, m), layer(xg))]
+        entry = layer.gemm_entry(m, xg)  # forward's own lookup
+        assert entry is None and m == 4096 or entry[0] == "tiled", entry  # what forward runs past the ladder
+        runs = [("rule", entry, layer(xg))]
         if m == 4096:  # the fused path at prefill size: x through the LDS ring, and both tiles through LDS
             for cfg in ((8, 2, 4, 1, 2, 1), (8, 4, 4, 2, 3, 1), (16, 4, 4, 1, 3, 0)):
                 runs.append(("forced gemm", cfg, ext.w4_gemm(xg, layer.packed, layer.scales, layer.zeros, buf, locks,
@@ -106,7 +106,7 @@ def test_qwen3_8b_prefill_sizes(proj, silu):
         for what, cfg, y in runs:
             assert y.shape == (m, n_out)
             got = y[:, torch.from_numpy(feats).to(DEV)].float().cpu().numpy()
-            kern = "dequant+matmul" if cfg is None else ("mma" if cfg[0] == "mma" else f"gemm s{cfg[4]}")
+            kern = "dequant+matmul" if cfg is None else (cfg[0] if cfg[0] in ("mma", "tiled") else f"gemm s{cfg[4]}")
             check_close(got, ref, 0.03 if silu else 0.05, 0.02, (proj, m, what, cfg), kern,
                         f"{proj}{'+silu' if silu else ''}")
         del xg, runs
