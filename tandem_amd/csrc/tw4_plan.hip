@@ -147,9 +147,10 @@ extern "C" int tw4_gemm_plan(int M, int N, int K, int act, int cus, int* out) {
             const int bm = 16 * p.mt * p.wm, bn = 16 * p.nt * p.wn;
             const int64_t tiles = cdiv(M, bm) * cdiv(N, bn);
             for (const int s : kPlanSplits)
-                if (split_ok(tiles, s, bm, bn))
-                    offer(std::max(floor, tile_cost(p.c, p.occ, bm, bn, tiles, 2 * cdiv(groups, s), s)),
-                          {3, p.mt, p.nt, p.wn, p.wm, p.wk, p.ring, s});
+                if (split_ok(tiles, s, bm, bn)) {
+                    const double t = tile_cost(p.c, p.occ, bm, bn, tiles, 2 * cdiv(groups, s), s);
+                    offer(std::max(floor, t) + 1e-3 * t, {3, p.mt, p.nt, p.wn, p.wm, p.wk, p.ring, s});  // at the floor: the least
+                }
         }
     if (M <= kPlanRingRows || !ints)  // past it only where nothing else takes the sizes
         for (const PlanRing& p : kPlanRing) {

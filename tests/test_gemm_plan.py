@@ -61,7 +61,7 @@ def _cheapest(m: int, n: int, k: int, act: int, cus: int) -> dict[tuple | None, 
             t[6:] = [v * scale for v in t[6:]]
             us = sum(a * b for a, b in zip(ROWS[cfg], t))
             if cfg[0] == "tiled":
-                us = max(us, 2.0 * m * n * k / 1.24e9 * scale)
+                us = max(us, 2.0 * m * n * k / 1.24e9 * scale) + 1e-3 * us
             costs[(*cfg, s) if cfg[0] == "tiled" else (*cfg[1:], s)] = us
     if m >= bench.FIT_DENSE_ROWS:
         t = bench.fit_terms(("dense",), m, n, k, act, 1, cus)
