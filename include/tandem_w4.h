@@ -185,9 +185,10 @@ int tw4_mma_persist(const uint16_t* x, const int32_t* packed, const uint16_t* sc
  *           prefetch chunk (1 or 2) and warps_k the wavefronts splitting each unit's groups (4 or 8);
  *           splits = 0 picks enough K splits to give every CU a unit
  *           3: large M: x AND the int4 weight tiles staged through LDS by direct-to-LDS loads
- *           (global_load_lds_dwordx4) in a 3-deep ring of half-group (64 k) stages; warps_k is then
+ *           (buffer_load_dwordx4 ... lds) in a ring of 3 half-group (64 k) stages (mt = nt = 8: 4); warps_k is then
  *           the number of wavefronts along M (BM = 16 mt warps_k, BN = 16 nt warps_n); N % 16 == 0,
- *           scales and zeros 16-byte aligned; splits = 0 picks enough K splits to fill the GPU
+ *           scales and zeros 16-byte aligned, M K < 2^31 and padded N K < 2^33; splits = 0 picks enough K splits
+ *           (ranges of whole quant groups) to fill the GPU
  *   splits  0: split only the last, partial wave of tiles along K; 1: no split; s > 1: every
  *           tile split s ways. The partial-wave rule counts tile waves, not bytes: where the whole
  *           grid fits in one wave it splits every tile, and on a bandwidth-bound shape the fp32

@@ -24,9 +24,11 @@
 //   split-K: work units (tile, split) take contiguous ranges of whole groups; the epilogue is the other GEMM's
 //            finish_unit (deterministic last-arriver reduction, counters returned to zero).
 //
-// What bounds it. Long calls (M N K from about 2^36): the matrix core, at the clock the card's power allows (1.7-1.9 GHz
-// under this load); 1.24 PFLOP/s against 1.3-1.5 of hipBLASLt's fp16 product without the dequantization. A wavefront
-// issues in order, about one instruction in 4 cycles, and an MFMA takes 16: the loop is software-pipelined in registers
+// What bounds it. Long calls (M N K from about 2^36): the matrix cores with the dequantization beside them, at the clock the
+// card's power allows: Qwen3-8B gate_up (4096 x 24576) at M = 4096 on 128 x 256 keeps them busy 67 % of the cycles, the VALU 51 %,
+// at 1.6 GHz (52 % and 37 % at 1.9-2.1 GHz before the pipeline below); 17 % of a CU's cycles go to LDS bank
+// conflicts. 1.24 PFLOP/s against 1.3-1.5 of hipBLASLt's fp16 product without the dequantization.
+// A wavefront issues in order, about one instruction in 4 cycles, and an MFMA takes 16: the loop is software-pipelined in registers
 // (the next fragments are read and the next weights dequantized between the current MFMAs, substep below), where a
 // read - dequantize - multiply sequence per substep left the matrix core idle for the first two. Short calls: the wait
 // for the first stages, the number of stages a CU runs in a row and how evenly the tiles divide over the CUs, hence the
@@ -385,7 +387,8 @@ gemm_lds_kernel(const h1* __restrict__ x, const u4* __restrict__ w, const h1* __
                                  m0 + wm * 16 * MT, tile0 + wn * NT, tiles_n, act);
 }
 
-// Compiled configurations (MT, NT, WM, WN, WK, ring slots): tw4_gemm's stages-3 ones, and the others of tw4_gemm_tiled.
+// Compiled configurations (MT, NT, WM, WN, WK, ring slots): tw4_gemm's stages-3 ones, and the others of tw4_gemm_tiled. Of the
+// first list the rule takes (8, 4, 1, 4, 1, 3) only; the rest are there for ladders that callers name them in.
 #define TW4_LDS_GEMM_CONFIGS(X) X(8, 4, 2, 4, 1, 3) X(16, 4, 1, 4, 1, 3) X(4, 4, 2, 4, 1, 3) X(8, 4, 2, 2, 1, 3) \
     X(8, 8, 1, 4, 1, 4) X(8, 4, 1, 4, 1, 3)
 #define TW4_TILED_GEMM_CONFIGS(X) X(8, 6, 2, 2, 1, 3) X(8, 6, 1, 2, 2, 4) X(8, 4, 1, 2, 2, 4) X(8, 3, 1, 2, 2, 4) \
