@@ -316,8 +316,9 @@ class W4Linear(nn.Module):
         if not isinstance(ladder, RuleLadder) or (ladder and m <= ladder[-1][0]):
             return pick_gemm(ladder, m)
         cfg = w4_plan.choose(m, self.out_features, self.in_features, self.silu_mul, self.cus)
-        if x is not None and w4_hip.intercepted():
-            return None if m > ladder.fused_rows else cfg or pick_gemm(DEFAULT_GEMM, min(m, 1024))
+        # up to fused_rows a kernel of the rule's is right whoever follows the call: the common case asks nothing more
+        if x is not None and (cfg is None or m > ladder.fused_rows) and w4_hip.intercepted():
+            return None if m > ladder.fused_rows else pick_gemm(DEFAULT_GEMM, min(m, 1024))
         return cfg
 
     def kernel_for(self, m: int) -> str:

@@ -504,11 +504,12 @@ def plain(x: torch.Tensor) -> bool:
             and (forward_ad._current_level < 0 or forward_ad.unpack_dual(x).tangent is None))
 
 
-def intercepted() -> bool:
+def intercepted(product: bool = True) -> bool:
     """Whether a torch operator called here would come out otherwise than by its arguments: autocast to another type than
     float16 gives a product another dtype, a torch function mode sees or replaces it (a default device does neither), a
-    compiler puts it into its graph. A call that was a torch operator stays one there; one that was a kernel stays a kernel."""
-    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.float16:
+    compiler puts it into its graph. A call that was a torch operator stays one there; one that was a kernel stays a kernel.
+    product: it is a product, which autocast takes part in."""
+    if product and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.float16:
         return True
     if torch._C._len_torch_function_stack() and any(not isinstance(mode, DeviceContext)
                                                     for mode in _get_current_function_mode_stack()):

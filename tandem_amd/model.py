@@ -105,7 +105,7 @@ class Attention(nn.Module):
         """Plain contiguous 16-byte aligned fp16 GPU rows [q | k | v] that no gradient, transform, mode or compiler follows, whole
         16-byte chunks per head: tw4_attend_one; anything else the torch expression of the same copy. One row with a KV
         head for each query head is no copy at all: its value columns as they lie."""
-        return (w4_hip.plain(qkv) and not w4_hip.intercepted() and qkv.is_cuda and qkv.dtype == torch.float16
+        return (w4_hip.plain(qkv) and not w4_hip.intercepted(product=False) and qkv.is_cuda and qkv.dtype == torch.float16
                 and qkv.dim() == 2 and qkv.numel() > 0 and qkv.is_contiguous()
                 and not (qkv.shape[0] == 1 and self.num_heads == self.num_kv_heads)
                 and qkv.shape[1] == self.q_size + 2 * self.kv_size and self.head_dim % 8 == 0
