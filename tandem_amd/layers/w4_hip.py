@@ -23,6 +23,7 @@ import os
 import threading
 
 import torch
+from torch._C import _functorch, _is_tracing, _len_torch_dispatch_stack
 from torch.autograd import forward_ad
 from torch.overrides import _get_current_function_mode_stack
 from torch.utils._device import DeviceContext
@@ -494,13 +495,16 @@ def release_stream_workspace(stream: torch.cuda.Stream) -> None:
                 _stream_workspaces.pop(key, None)
 
 
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
+
+
 def plain(x: torch.Tensor) -> bool:
     """An ordinary tensor that only the values of this call matter to: no gradient or tangent is asked of it, no transform
     (vmap, jvp), tracer or dispatch mode follows the call. Anything else has to stay in torch operators, as a kernel that
     sees a data pointer only would drop what follows it."""
-    return (type(x) in (torch.Tensor, torch.nn.Parameter) and not (x.requires_grad and torch.is_grad_enabled())
-            and not torch._C._is_tracing() and not torch._C._len_torch_dispatch_stack()
-            and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+    return (type(x) in _TENSORS and not (x.requires_grad and torch.is_grad_enabled())
+            and not _is_tracing() and not _len_torch_dispatch_stack()
+            and (_functorch.peek_interpreter_stack() is None or not _functorch.is_functorch_wrapped_tensor(x))
             and (forward_ad._current_level < 0 or forward_ad.unpack_dual(x).tangent is None))
 
 
