@@ -215,7 +215,7 @@ int tw4_gemm(const uint16_t* x, const int32_t* packed, const uint16_t* scales,
  * N % 8 == 0 with scales and zeros 4-byte aligned. BM = 16 mt warps_m tokens, BN = 16 nt warps_n rows, `ring` stages
  * of 64 k in LDS, warps_k 1, or 2: two wavefronts per (tokens, rows) part, each with half of every stage. splits: 0 as
  * for stages 3, 1, or that many contiguous ranges of whole quant groups per tile (at most 2 K / 128; a range past the
- * groups is empty). Otherwise tw4_gemm's contract. No reference counterpart beyond
+ * groups is empty). M K < 2^31 and padded N K < 2^33 (32-bit load offsets). Otherwise tw4_gemm's contract. No reference counterpart beyond
  * w4_gemm's (python/tandem/csrc/w4_gemv.cu:312-566). */
 int tw4_gemm_tiled(const uint16_t* x, const int32_t* packed, const uint16_t* scales,
                    const uint16_t* zeros, uint16_t* y, float* ws, int32_t* locks,
