@@ -15,7 +15,9 @@ typedef __attribute__((address_space(3))) const void lds_void;
 // after it is written (the M0 -> LDS-DMA hazard).
 // The 16-byte form goes through a buffer resource: the part of the address that moves with the stage is one 32-bit
 // scalar offset, the lane's own offset is fixed for the whole kernel, and a resource of no records turns the load into
-// one that reads nothing (zeros), which is how the stages past the end keep the loop's counts without a branch.
+// one that reads nothing (zeros), which is how the stages past the end keep the loop's counts without a branch: the range
+// check takes lane and scalar offset together, whatever the scalar one (no records at an offset of 4 KB: zeros; 4608 bytes: the first
+// 512 from there).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"  // m0 is a reserved register: the clobber is what tells the compiler
 template <int IMM, bool NT = false>  // NT: non-temporal, data that is read once
